@@ -29,6 +29,8 @@ struct Plan {
     int j = 0;            // chunks held per lane (x registers)
     int r = 0;            // rows per lane
     int tile = 0;         // chunks per lane per tile (K-tiled kernels), else 0
+    int split = 0;        // waves sharing a row (scalar kernels), else 0
+    int batch = 0;        // chunks per lane per batch (scalar kernels), else 0
     int block = 0;        // threads per workgroup
     int64_t grid = 0;     // workgroups
     bool fallback = false;  // requested a wave variant, got the scalar kernel

@@ -9,11 +9,11 @@
 //
 // Two kernel families per operator:
 //
-// * scalar (`*_scalar_kernel`): one 256-thread workgroup per row, strided
-//   1-byte weight loads, per-element dequant `fma(q*s, x, acc)`, DPP wave
-//   reduction, LDS across the 4 waves.  It has no alignment requirement and
-//   is the single source for the *_baseline variants and for every
-//   fallback (bit-identity of fallback and baseline follows from that).
+// * scalar (`*_scalar_kernel`): 16-byte loads of any alignment, any k,
+//   per-element dequant `fma(q*s, x, acc)`, DPP wave reduction, LDS across
+//   the waves that share a row.  It is the single source for the *_baseline
+//   variants and for every fallback (bit-identity of fallback and baseline
+//   follows from that and from a plan that depends on the sizes alone).
 //
 // * wave (`*_wave_kernel<CW, J, R>`): the CDNA4 design.
 //   - Lanes of a wave64 are split into 64/CW row slots of CW lanes; lane
@@ -113,52 +113,277 @@ __device__ __forceinline__ uint32_t xcd_contiguous_block() {
 }
 
 // ---------------------------------------------------------------- scalar
+//
+// The kernels of the *_baseline variants and of every call that misses the
+// vector contract (any alignment, any k): per-element arithmetic, as the
+// reference's scalar kernels define it (INT4/INT8 fma(float(q) * s, x, acc),
+// FP16/FP32 fma(w, x, acc)), on 16-byte loads that need no alignment.
+//
+// SP waves share R rows.  Lane `lane` of the i-th of them owns the 16-byte
+// weight chunks lane + 64 (i + SP j) of a row (E elements each) and loads x
+// for them straight from memory (every wave reads x, so it sits in the
+// caches), once for its R rows.  Batches of U chunks run through two register
+// sets: batch b + 1 is in flight while batch b is summed.  The k % E elements
+// past the last whole chunk go one per lane.  Four accumulators per lane keep
+// the FMA chains as short as one element per thread of a 256-thread workgroup
+// would; the shares of a row meet in LDS and are added in wave order.  Chunks
+// past the row end are re-read in bounds and not summed (no zero operand
+// stands in for them, so an infinite scale or x meets no extra product).
+//
+// Bound by memory.  With one element per load and one workgroup per row (the
+// form before) the memory system was idle: INT8 4001x4099 (16 MB) 12.2 us,
+// now 6.3; FP16 4096^2 off alignment 18.3 us, now 8.0.  What is left of the
+// distance to the aligned kernels (INT8 4096^2 4.4 us) is the loads that
+// start off a 4-byte boundary: the same INT8 4096^2 call on this kernel is
+// 5.3 us with W 4 or 8 bytes off, 6.0 with W 1 or 2 bytes off.
 
-__global__ __launch_bounds__(kBlock) void int4gemv_scalar_kernel(
-        const uint8_t* __restrict__ w, const uint16_t* __restrict__ scale,
-        const uint16_t* __restrict__ x, uint16_t* __restrict__ y,
-        int64_t k) {
-    const int64_t row = blockIdx.x;
-    const int64_t kb = k >> 1;  // bytes per row
-    const uint8_t* __restrict__ wrow = w + row * kb;
-    const uint16_t* __restrict__ srow = scale + row * (k >> 7);
-    float acc = 0.f;
-    for (int64_t b = threadIdx.x; b < kb; b += kBlock) {
-        const uint32_t byte = wrow[b];
-        const float s = h2f(srow[b >> 6]);  // both nibbles: group b/64
-        // sign-extend bits 0-3 (element 2b) and bits 4-7 (element 2b+1)
-        const int32_t lo = static_cast<int32_t>(byte << 28) >> 28;
-        const int32_t hi = static_cast<int32_t>(byte << 24) >> 28;
-        acc = __builtin_fmaf(static_cast<float>(lo) * s, h2f(x[2 * b]), acc);
-        acc = __builtin_fmaf(static_cast<float>(hi) * s, h2f(x[2 * b + 1]),
-                             acc);
-    }
-    acc = segment_sum<64>(acc);
-    __shared__ float part[kBlock / 64];
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    if (lane == 63) part[wave] = acc;
-    __syncthreads();
-    if (threadIdx.x == 0) y[row] = f2h((part[0] + part[1]) + (part[2] + part[3]));
+__device__ __forceinline__ uint4 load16_any(const char* p) {
+    uint4 v;
+    __builtin_memcpy(&v, p, 16);
+    return v;
 }
 
-__global__ __launch_bounds__(kBlock) void qgemv_scalar_kernel(
-        const int8_t* __restrict__ w, const float* __restrict__ scale,
-        const uint16_t* __restrict__ x, uint16_t* __restrict__ y,
-        int64_t k) {
-    const int64_t row = blockIdx.x;
-    const int8_t* __restrict__ wrow = w + row * k;
-    const float s = scale[row];
-    float acc = 0.f;
-    for (int64_t i = threadIdx.x; i < k; i += kBlock)
-        acc = __builtin_fmaf(static_cast<float>(wrow[i]) * s, h2f(x[i]), acc);
-    acc = segment_sum<64>(acc);
-    __shared__ float part[kBlock / 64];
+// float(q) * s for a value held exactly in fp16: one v_fma_mix_f32.  Adding
+// -0 changes no product, signed zeros included.
+__device__ __forceinline__ float times_scale(_Float16 q, float s) {
+    return __builtin_fmaf(static_cast<float>(q), s, -0.0f);
+}
+
+// Per operator: E elements per 16-byte chunk, XP 16-byte pieces of x per
+// chunk, `Scale` what a chunk needs to be summed, `sum` one chunk into the
+// four accumulators, `one` a single element.
+struct AnyInt4 {
+    using Y = uint16_t;
+    static constexpr int E = 32, XP = 4, kXBytes = 2;
+    static constexpr bool kGroupScale = true;
+    static __device__ __forceinline__ float scale_of(const void* s, int64_t, int64_t i) {
+        return h2f(static_cast<const uint16_t*>(s)[i]);
+    }
+    static __device__ __forceinline__ void sum(const uint4& w, const uint4 (&x)[XP],
+                                               float s, float (&acc)[4]) {
+        const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
+        const f16x2 bias_lo = {static_cast<_Float16>(-1032.0f), static_cast<_Float16>(-1032.0f)};
+        const f16x2 bias_hi = {static_cast<_Float16>(-72.0f), static_cast<_Float16>(-72.0f)};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t u = ws[i], u8 = u >> 8;
+            const f16x2 x01 = as_f16x2(x[i].x), x23 = as_f16x2(x[i].y);
+            const f16x2 x45 = as_f16x2(x[i].z), x67 = as_f16x2(x[i].w);
+            // pairs (q0, q4), (q1, q5), (q2, q6), (q3, q7)
+            const f16x2 qa = as_f16x2((u & 0x000F000Fu) ^ 0x64086408u) + bias_lo;
+            const f16x2 qb = as_f16x2((u & 0x00F000F0u) ^ 0x54805480u) + bias_hi;
+            const f16x2 qc = as_f16x2((u8 & 0x000F000Fu) ^ 0x64086408u) + bias_lo;
+            const f16x2 qd = as_f16x2((u8 & 0x00F000F0u) ^ 0x54805480u) + bias_hi;
+            acc[0] = __builtin_fmaf(times_scale(qa[0], s), static_cast<float>(x01[0]), acc[0]);
+            acc[1] = __builtin_fmaf(times_scale(qb[0], s), static_cast<float>(x01[1]), acc[1]);
+            acc[2] = __builtin_fmaf(times_scale(qc[0], s), static_cast<float>(x23[0]), acc[2]);
+            acc[3] = __builtin_fmaf(times_scale(qd[0], s), static_cast<float>(x23[1]), acc[3]);
+            acc[0] = __builtin_fmaf(times_scale(qa[1], s), static_cast<float>(x45[0]), acc[0]);
+            acc[1] = __builtin_fmaf(times_scale(qb[1], s), static_cast<float>(x45[1]), acc[1]);
+            acc[2] = __builtin_fmaf(times_scale(qc[1], s), static_cast<float>(x67[0]), acc[2]);
+            acc[3] = __builtin_fmaf(times_scale(qd[1], s), static_cast<float>(x67[1]), acc[3]);
+        }
+    }
+    // k % 128 == 0: no element past the last whole chunk
+    static __device__ __forceinline__ float one(const char*, const char*, int64_t, float,
+                                                float acc) { return acc; }
+    static __device__ __forceinline__ void store(Y* y, float v) { *y = f2h(v); }
+};
+
+struct AnyInt8 {
+    using Y = uint16_t;
+    static constexpr int E = 16, XP = 2, kXBytes = 2;
+    static constexpr bool kGroupScale = false;
+    static __device__ __forceinline__ float scale_of(const void* s, int64_t row, int64_t) {
+        return static_cast<const float*>(s)[row];
+    }
+    static __device__ __forceinline__ void sum(const uint4& w, const uint4 (&x)[XP],
+                                               float s, float (&acc)[4]) {
+        const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
+        const uint32_t xw[8] = {x[0].x, x[0].y, x[0].z, x[0].w, x[1].x, x[1].y, x[1].z, x[1].w};
+        const f16x2 bias = {static_cast<_Float16>(-1152.0f), static_cast<_Float16>(-1152.0f)};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t u = ws[i];
+            // pairs (q0, q2), (q1, q3)
+            const f16x2 qa = as_f16x2((u & 0x00FF00FFu) ^ 0x64806480u) + bias;
+            const f16x2 qb = as_f16x2(((u >> 8) & 0x00FF00FFu) ^ 0x64806480u) + bias;
+            const f16x2 x01 = as_f16x2(xw[2 * i]), x23 = as_f16x2(xw[2 * i + 1]);
+            acc[0] = __builtin_fmaf(times_scale(qa[0], s), static_cast<float>(x01[0]), acc[0]);
+            acc[1] = __builtin_fmaf(times_scale(qb[0], s), static_cast<float>(x01[1]), acc[1]);
+            acc[2] = __builtin_fmaf(times_scale(qa[1], s), static_cast<float>(x23[0]), acc[2]);
+            acc[3] = __builtin_fmaf(times_scale(qb[1], s), static_cast<float>(x23[1]), acc[3]);
+        }
+    }
+    static __device__ __forceinline__ float one(const char* w, const char* x, int64_t i,
+                                                float s, float acc) {
+        const float q = static_cast<float>(reinterpret_cast<const int8_t*>(w)[i]);
+        return __builtin_fmaf(q * s, h2f(reinterpret_cast<const uint16_t*>(x)[i]), acc);
+    }
+    static __device__ __forceinline__ void store(Y* y, float v) { *y = f2h(v); }
+};
+
+struct AnyF16 {
+    using Y = uint16_t;
+    static constexpr int E = 8, XP = 1, kXBytes = 2;
+    static constexpr bool kGroupScale = false;
+    static __device__ __forceinline__ float scale_of(const void*, int64_t, int64_t) { return 0.f; }
+    static __device__ __forceinline__ void sum(const uint4& w, const uint4 (&x)[XP], float,
+                                               float (&acc)[4]) {
+        const uint32_t ws[4] = {w.x, w.y, w.z, w.w}, xw[4] = {x[0].x, x[0].y, x[0].z, x[0].w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const f16x2 a = as_f16x2(ws[i]), b = as_f16x2(xw[i]);
+            acc[i] = __builtin_fmaf(static_cast<float>(a[0]), static_cast<float>(b[0]), acc[i]);
+            acc[i] = __builtin_fmaf(static_cast<float>(a[1]), static_cast<float>(b[1]), acc[i]);
+        }
+    }
+    static __device__ __forceinline__ float one(const char* w, const char* x, int64_t i, float,
+                                                float acc) {
+        return __builtin_fmaf(h2f(reinterpret_cast<const uint16_t*>(w)[i]),
+                              h2f(reinterpret_cast<const uint16_t*>(x)[i]), acc);
+    }
+    static __device__ __forceinline__ void store(Y* y, float v) { *y = f2h(v); }
+};
+
+struct AnyF32 {
+    using Y = float;
+    static constexpr int E = 4, XP = 1, kXBytes = 4;
+    static constexpr bool kGroupScale = false;
+    static __device__ __forceinline__ float scale_of(const void*, int64_t, int64_t) { return 0.f; }
+    static __device__ __forceinline__ void sum(const uint4& w, const uint4 (&x)[XP], float,
+                                               float (&acc)[4]) {
+        const uint32_t ws[4] = {w.x, w.y, w.z, w.w}, xw[4] = {x[0].x, x[0].y, x[0].z, x[0].w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            acc[i] = __builtin_fmaf(__builtin_bit_cast(float, ws[i]),
+                                    __builtin_bit_cast(float, xw[i]), acc[i]);
+    }
+    static __device__ __forceinline__ float one(const char* w, const char* x, int64_t i, float,
+                                                float acc) {
+        return __builtin_fmaf(reinterpret_cast<const float*>(w)[i],
+                              reinterpret_cast<const float*>(x)[i], acc);
+    }
+    static __device__ __forceinline__ void store(Y* y, float v) { *y = v; }
+};
+
+template <class Op, int R, int U, int SP>
+__device__ __forceinline__ void scalar_rows(
+        const char* __restrict__ w,      // [n][k] elements, any alignment
+        const void* __restrict__ scale,  // INT4 [n][k/128], INT8 [n], else unused
+        const char* __restrict__ x,      // [k]
+        typename Op::Y* __restrict__ y, int n, int64_t k) {
+    constexpr int E = Op::E, XP = Op::XP;
+    constexpr int64_t kXStep = 64 * E * Op::kXBytes;    // x bytes of 64 chunks
     const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    if (lane == 63) part[wave] = acc;
-    __syncthreads();
-    if (threadIdx.x == 0) y[row] = f2h((part[0] + part[1]) + (part[2] + part[3]));
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int part = wave % SP;                // this wave's share of its rows' chunks
+    const int64_t row0 = (static_cast<int64_t>(xcd_contiguous_block()) * (kBlock / 64 / SP) +
+                          wave / SP) * R;
+    const int64_t nfull = k / E;               // whole chunks of a row
+    const int64_t niter = (nfull + 63) / 64;   // 64 chunks each; this wave takes part + SP i
+    const int64_t wrow_bytes = nfull * 16 + (k - nfull * E) * (16 / E);
+    const int64_t groups = k / 128;
+    const char* wr[R];
+    float srow[R];
+    int64_t rows[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        rows[r] = std::min<int64_t>(row0 + r, n - 1);
+        wr[r] = w + rows[r] * wrow_bytes;
+        srow[r] = Op::kGroupScale ? 0.f : Op::scale_of(scale, rows[r], 0);
+    }
+    struct Batch {
+        uint4 w[R][U];
+        uint4 x[U][XP];
+        float s[R][U];
+    };
+    auto load = [&](Batch& b, int64_t it0) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            // wave-uniform bases; iterations past the last re-read it, lanes
+            // past the row end re-read its last chunk
+            const int64_t it = std::min<int64_t>(it0 + SP * u, niter - 1);
+            const int last = static_cast<int>(std::min<int64_t>(63, nfull - 1 - 64 * it));
+            const uint32_t l = static_cast<uint32_t>(std::min(lane, last));
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                b.w[r][u] = load16_any(wr[r] + it * 1024 + l * 16u);
+                b.s[r][u] = Op::kGroupScale
+                    ? Op::scale_of(scale, 0, rows[r] * groups + it * 16 + (l >> 2)) : srow[r];
+            }
+            const char* xp = x + it * kXStep + l * static_cast<uint32_t>(16 * XP);
+#pragma unroll
+            for (int p = 0; p < XP; ++p) b.x[u][p] = load16_any(xp + 16 * p);
+        }
+    };
+    float acc[R][4] = {};
+    auto sum = [&](const Batch& b, int64_t it0) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if ((it0 + SP * u) * 64 + lane < nfull)
+#pragma unroll
+                for (int r = 0; r < R; ++r) Op::sum(b.w[r][u], b.x[u], b.s[r][u], acc[r]);
+    };
+    if (part < niter) {
+        constexpr int64_t kStep = SP * U;
+        Batch b0, b1;
+        load(b0, part);
+        for (int64_t it = part; it < niter; it += 2 * kStep) {
+            if (it + kStep < niter) load(b1, it + kStep);
+            sum(b0, it);
+            if (it + kStep < niter) {
+                if (it + 2 * kStep < niter) load(b0, it + 2 * kStep);
+                sum(b1, it + kStep);
+            }
+        }
+    }
+    // the elements past the last whole chunk, one per lane, by the last wave
+    const int64_t tail = nfull * E + lane;
+    if (part == SP - 1 && tail < k)
+#pragma unroll
+        for (int r = 0; r < R; ++r) acc[r][0] = Op::one(wr[r], x, tail, srow[r], acc[r][0]);
+    float a[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+        a[r] = segment_sum<64>((acc[r][0] + acc[r][1]) + (acc[r][2] + acc[r][3]));
+    if constexpr (SP > 1) {
+        __shared__ float shares[kBlock / 64][R];
+        if (lane == 63)
+#pragma unroll
+            for (int r = 0; r < R; ++r) shares[wave][r] = a[r];
+        __syncthreads();
+        if (part != 0) return;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            a[r] = shares[wave][r];
+#pragma unroll
+            for (int i = 1; i < SP; ++i) a[r] += shares[wave + i][r];
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+        if (lane == 63 && row0 + r < n) Op::store(y + row0 + r, a[r]);
+}
+
+template <int R, int U, int SP>
+__global__ __launch_bounds__(kBlock) void int4gemv_scalar_kernel(
+        const char* __restrict__ w, const void* __restrict__ scale,
+        const char* __restrict__ x, uint16_t* __restrict__ y, int n, int64_t k) {
+    scalar_rows<AnyInt4, R, U, SP>(w, scale, x, y, n, k);
+}
+template <int R, int U, int SP>
+__global__ __launch_bounds__(kBlock) void qgemv_scalar_kernel(
+        const char* __restrict__ w, const void* __restrict__ scale,
+        const char* __restrict__ x, uint16_t* __restrict__ y, int n, int64_t k) {
+    scalar_rows<AnyInt8, R, U, SP>(w, scale, x, y, n, k);
+}
+template <typename S, int R, int U, int SP>
+__global__ __launch_bounds__(kBlock) void gemv_scalar_kernel(
+        const char* __restrict__ w, const void* __restrict__ scale,
+        const char* __restrict__ x, S* __restrict__ y, int n, int64_t k) {
+    scalar_rows<std::conditional_t<sizeof(S) == 4, AnyF32, AnyF16>, R, U, SP>(
+        w, scale, x, y, n, k);
 }
 
 // ------------------------------------------------------------------ wave
@@ -1004,8 +1229,6 @@ __global__ __launch_bounds__(NT) void qgemv_lds_group_kernel(GroupArgs g,
 // y[n] = sum_k W[n,k] * x[k] accumulated in FP32 and cast once to the
 // dtype of W (RNE for fp16).  W and x are fp16 or fp32, same dtype.
 
-__device__ __forceinline__ float fp_to_f(uint16_t h) { return h2f(h); }
-__device__ __forceinline__ float fp_to_f(float f) { return f; }
 __device__ __forceinline__ void fp_store(uint16_t* p, float v) { *p = f2h(v); }
 __device__ __forceinline__ void fp_store(float* p, float v) { *p = v; }
 
@@ -1037,26 +1260,6 @@ __device__ __forceinline__ void dot_chunk(float, const uint4& w,
     acc[1] = __builtin_fmaf(__builtin_bit_cast(float, w.y), __builtin_bit_cast(float, x.y), acc[1]);
     acc[2] = __builtin_fmaf(__builtin_bit_cast(float, w.z), __builtin_bit_cast(float, x.z), acc[2]);
     acc[3] = __builtin_fmaf(__builtin_bit_cast(float, w.w), __builtin_bit_cast(float, x.w), acc[3]);
-}
-
-// Scalar: one 256-thread workgroup per row, element loads.  The single
-// source of gemv_baseline and of every fallback (bit-identity of the two).
-template <typename S>
-__global__ __launch_bounds__(kBlock) void gemv_scalar_kernel(
-        const S* __restrict__ w, const S* __restrict__ x, S* __restrict__ y,
-        int64_t k) {
-    const int64_t row = blockIdx.x;
-    const S* __restrict__ wrow = w + row * k;
-    float acc = 0.f;
-    for (int64_t i = threadIdx.x; i < k; i += kBlock)
-        acc = __builtin_fmaf(fp_to_f(wrow[i]), fp_to_f(x[i]), acc);
-    acc = segment_sum<64>(acc);
-    __shared__ float part[kBlock / 64];
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    if (lane == 63) part[wave] = acc;
-    __syncthreads();
-    if (threadIdx.x == 0) fp_store(y + row, (part[0] + part[1]) + (part[2] + part[3]));
 }
 
 // Vector: CW lanes per row (64/CW rows per wave), lane `col` owns the
@@ -1415,6 +1618,28 @@ hipError_t bind(Launch* out, void (*kernel)(Params...), int64_t grid,
     return hipSuccess;
 }
 
+// Instances of the scalar kernels that scalar_plan can ask for.
+struct Int4Scalar {
+    template <int R, int U, int SP>
+    static constexpr auto get() { return &int4gemv_scalar_kernel<R, U, SP>; }
+};
+struct Q8Scalar {
+    template <int R, int U, int SP>
+    static constexpr auto get() { return &qgemv_scalar_kernel<R, U, SP>; }
+};
+template <typename S>
+struct GemvScalar {
+    template <int R, int U, int SP>
+    static constexpr auto get() { return &gemv_scalar_kernel<S, R, U, SP>; }
+};
+template <class F>
+auto scalar_instance(const Plan& p) {
+    if (p.split == 1) return p.r == 1 ? F::template get<1, 1, 1>() : F::template get<2, 1, 1>();
+    if (p.split == 2) return p.r == 1 ? F::template get<1, 1, 2>() : F::template get<2, 1, 2>();
+    if (p.batch == 1) return p.r == 1 ? F::template get<1, 1, 4>() : F::template get<2, 1, 4>();
+    return p.r == 1 ? F::template get<1, 2, 4>() : F::template get<2, 2, 4>();
+}
+
 int pow2_at_least(int64_t v, int lo) {
     int p = lo;
     while (p < v && p < 64) p <<= 1;
@@ -1484,11 +1709,28 @@ void finish_wave_plan(Plan& p, int64_t n, bool int4) {
     p.grid = (waves + block_waves - 1) / block_waves;
 }
 
-Plan scalar_plan(int64_t n, bool fallback, const char* why) {
+// Plan of the scalar kernels, from the sizes alone (so that a call off the
+// vector contract and the same call of a *_baseline variant sum in the same
+// order).  `per` is the elements of a 16-byte chunk.  A row is `steps` rounds
+// of 64 chunks; measured over HBM-cold pools (us per call):
+// - waves per row: 1 for one step (INT8 32000x333: 8.7; 2 waves 10.2, 4 14.8),
+//   2 for two or three (INT4 4096^2 5.0; 1 wave 6.2, 4 5.6), 4 from there
+//   (INT8 1000x30001 11.0; 1 wave 27, 2 15.7);
+// - rows per wave: 2 (INT8 4001x4099 6.3; 1 row 6.9), but 1 up to 512 rows,
+//   where two would leave CUs idle (FP32 500x5001 4.4 against 4.6, INT8
+//   256x4099 2.4 against 2.9);
+// - chunks per batch: 2 from 16 steps (INT8 300x131071 18.9, one chunk 25.4),
+//   else 1 (INT8 4001x4099 with two: 8.6).
+Plan scalar_plan(int64_t n, int64_t k, int per, bool fallback, const char* why) {
     Plan p;
     p.kind = kScalar;
     p.block = kBlock;
-    p.grid = n;
+    const int64_t steps = (k / per + 63) / 64;
+    p.split = steps <= 1 ? 1 : steps <= 3 ? 2 : 4;
+    p.batch = steps >= 16 ? 2 : 1;
+    p.r = n <= 512 ? 1 : 2;
+    const int64_t rows = p.r * (kBlock / 64 / p.split);    // per workgroup
+    p.grid = (n + rows - 1) / rows;
     p.fallback = fallback;
     p.why = why;
     return p;
@@ -1531,16 +1773,16 @@ bool q8_contract_ok(const void* w, const void* x, int64_t k) {
 
 Plan plan_int4(int kind, int rows, int64_t n, int64_t k, const void* w,
                const void* x) {
-    if (kind == kScalar) return scalar_plan(n, false, "");
+    if (kind == kScalar) return scalar_plan(n, k, AnyInt4::E, false, "");
     if (!int4_contract_ok(w, x, k))
-        return scalar_plan(n, true, "vector contract unmet (w/x 16B alignment, k%32)");
+        return scalar_plan(n, k, AnyInt4::E, true, "vector contract unmet (w/x 16B alignment, k%32)");
     const int64_t nchunks = k / 32;
     // the untiled LDS kernels address W with 32-bit byte offsets; the tiled
     // kernel keeps 64-bit row bases, so it also takes weights of 4 GiB or more
     const bool big = n * (k / 2) >= (int64_t{1} << 32);
     if (kind == kTiled || (kind == kLds && (k > kMaxWaveK || big)))
         return tiled_plan(rows, n, nchunks, true);
-    if (k > kMaxWaveK) return scalar_plan(n, true, "k above the wave kernels' register-resident x");
+    if (k > kMaxWaveK) return scalar_plan(n, k, AnyInt4::E, true, "k above the wave kernels' register-resident x");
     Plan p;
     p.kind = kind;
     p.cw = pow2_at_least(nchunks, 16);
@@ -1554,14 +1796,14 @@ Plan plan_int4(int kind, int rows, int64_t n, int64_t k, const void* w,
 
 Plan plan_q8(int kind, int rows, int64_t n, int64_t k, const void* w,
              const void* x) {
-    if (kind == kScalar) return scalar_plan(n, false, "");
+    if (kind == kScalar) return scalar_plan(n, k, AnyInt8::E, false, "");
     if (!q8_contract_ok(w, x, k))
-        return scalar_plan(n, true, "vector contract unmet (w/x 16B alignment, k%16)");
+        return scalar_plan(n, k, AnyInt8::E, true, "vector contract unmet (w/x 16B alignment, k%16)");
     const int64_t nchunks = k / 16;
     const bool big = n * k >= (int64_t{1} << 32);    // as in plan_int4
     if (kind == kTiled || (kind == kLds && (k > kMaxWaveK || big)))
         return tiled_plan(rows, n, nchunks, false);
-    if (k > kMaxWaveK) return scalar_plan(n, true, "k above the wave kernels' register-resident x");
+    if (k > kMaxWaveK) return scalar_plan(n, k, AnyInt8::E, true, "k above the wave kernels' register-resident x");
     Plan p;
     p.kind = kind;
     p.cw = pow2_at_least(nchunks, 16);
@@ -1576,10 +1818,10 @@ Plan plan_q8(int kind, int rows, int64_t n, int64_t k, const void* w,
 hipError_t prepare_int4(const Plan& p, const void* w, const void* scale,
                         const void* x, void* y, int64_t n, int64_t k, Launch* L) {
     if (p.kind == kScalar)
-        return bind(L, int4gemv_scalar_kernel, p.grid, p.block, 0,
-                    static_cast<const uint8_t*>(w),
-                    static_cast<const uint16_t*>(scale),
-                    static_cast<const uint16_t*>(x), static_cast<uint16_t*>(y), k);
+        return bind(L, scalar_instance<Int4Scalar>(p),
+                    p.grid, p.block, 0, static_cast<const char*>(w), scale,
+                    static_cast<const char*>(x), static_cast<uint16_t*>(y),
+                    static_cast<int>(n), k);
     if (p.kind == kTiled) {
         const Int4Fn tfn =
             p.r == 1 && p.tile == 7   ? &int4gemv_tiled_kernel<kBlock, 7, 1>
@@ -1608,9 +1850,10 @@ hipError_t prepare_int4(const Plan& p, const void* w, const void* scale,
 hipError_t prepare_q8(const Plan& p, const void* w, const void* scale,
                       const void* x, void* y, int64_t n, int64_t k, Launch* L) {
     if (p.kind == kScalar)
-        return bind(L, qgemv_scalar_kernel, p.grid, p.block, 0,
-                    static_cast<const int8_t*>(w), static_cast<const float*>(scale),
-                    static_cast<const uint16_t*>(x), static_cast<uint16_t*>(y), k);
+        return bind(L, scalar_instance<Q8Scalar>(p),
+                    p.grid, p.block, 0, static_cast<const char*>(w), scale,
+                    static_cast<const char*>(x), static_cast<uint16_t*>(y),
+                    static_cast<int>(n), k);
     if (p.kind == kTiled) {
         const Q8Fn tfn = p.r == 2 && p.tile == q8_tile_j(2) ? &qgemv_tiled_kernel<kBlock, q8_tile_j(2), 2>
                          : p.r == 1 && p.tile == q8_tile_j(1) ? &qgemv_tiled_kernel<kBlock, q8_tile_j(1), 1>
@@ -1808,16 +2051,17 @@ bool gemv_contract_ok(int dtype, const void* w, const void* x, int64_t k) {
 
 Plan plan_gemv(int kind, int dtype, int64_t n, int64_t k, const void* w,
                const void* x) {
-    if (kind == kScalar) return scalar_plan(n, false, "");
+    const int per = dtype == kF32 ? AnyF32::E : AnyF16::E;
+    if (kind == kScalar) return scalar_plan(n, k, per, false, "");
     if (!gemv_contract_ok(dtype, w, x, k))
-        return scalar_plan(n, true, "vector contract unmet (w/x 16B alignment, k % elements per 16 B)");
+        return scalar_plan(n, k, per, true, "vector contract unmet (w/x 16B alignment, k % elements per 16 B)");
     const int64_t es = dtype == kF32 ? 4 : 2;
     const int64_t nchunks = k * es / 16;
     // in-row byte offsets are 32-bit in every vector kernel; row bases are
     // 64-bit only in the tiled kernel, which therefore also takes weights
     // of 4 GiB or more
     if (k * es >= (int64_t{1} << 32))
-        return scalar_plan(n, true, "rows of 4 GiB or more (32-bit offsets)");
+        return scalar_plan(n, k, per, true, "rows of 4 GiB or more (32-bit offsets)");
     const bool big = n * k * es >= (int64_t{1} << 32);
     Plan p;
     if (kind == kTiled || big || (nchunks + 1) * 16 > kGemvMaxLdsBytes) {
@@ -1875,9 +2119,8 @@ template <typename S>
 hipError_t prepare_gemv_t(const Plan& p, const void* w, const void* x, void* y,
                           int64_t n, int64_t k, Launch* L) {
     if (p.kind == kScalar)
-        return bind(L, gemv_scalar_kernel<S>, p.grid, p.block, 0,
-                    static_cast<const S*>(w), static_cast<const S*>(x),
-                    static_cast<S*>(y), k);
+        return bind(L, scalar_instance<GemvScalar<S>>(p), p.grid, p.block, 0,
+                    static_cast<const char*>(w), nullptr, static_cast<const char*>(x), static_cast<S*>(y), static_cast<int>(n), k);
     const int nchunks = static_cast<int>(k * static_cast<int64_t>(sizeof(S)) / 16);
     if (p.kind == kTiled)
         return bind(L, p.block == 512 ? gemv_tiled_kernel<S, 512> : gemv_tiled_kernel<S, kBlock>,
