@@ -96,6 +96,10 @@ SIGNATURES = {
                                         ctypes.c_int, _vp]),
     "cq_q8_quantize": (ctypes.c_int, [_vp, _vp, _vp, _i64, _i64,
                                       ctypes.c_int, _vp]),
+    "cq_int4_quantize_flagged": (ctypes.c_int, [_vp, _vp, _vp, _i64, _i64,
+                                                ctypes.c_int, _vp, _vp]),
+    "cq_q8_quantize_flagged": (ctypes.c_int, [_vp, _vp, _vp, _i64, _i64,
+                                              ctypes.c_int, _vp, _vp]),
     "cq_quantize_vectorized": (ctypes.c_int, [ctypes.c_int, _vp, _vp, _i64,
                                               _i64]),
     "cq_native_timing": (ctypes.c_int, [

@@ -284,7 +284,7 @@ int run_one(int op, const char* variant, const void* w, const void* scale,
 // Argument checks of the quantizer entry points (plain pointers and sizes;
 // the Python layer keeps the reference's ValueError checks on metadata).
 int check_quantize(int op, const void* w, const void* q, const void* scale,
-                   int64_t n, int64_t k, int scale_mode) {
+                   int64_t n, int64_t k, int scale_mode, const uint32_t* nonfinite) {
     if (scale_mode != CQ_SCALE_DIV && scale_mode != CQ_SCALE_RCP)
         return fail(CQ_ERR_INVALID_ARG, "unknown scale_mode " + std::to_string(scale_mode));
     if (w == nullptr || q == nullptr || scale == nullptr)
@@ -311,6 +311,15 @@ int check_quantize(int op, const void* w, const void* q, const void* scale,
     if (overlaps(in, o.w) || overlaps(in, o.scale) || overlaps(o.w, o.scale))
         return fail(CQ_ERR_INVALID_ARG, "w, the quantized output and scale must not "
                                         "overlap");
+    if (nonfinite != nullptr) {
+        Span f;
+        f.lo = reinterpret_cast<uintptr_t>(nonfinite);
+        f.hi = f.lo + sizeof *nonfinite;
+        if (f.lo % sizeof *nonfinite != 0)
+            return fail(CQ_ERR_INVALID_ARG, "the nonfinite word must be 4-byte aligned");
+        if (overlaps(f, in) || overlaps(f, o.w) || overlaps(f, o.scale))
+            return fail(CQ_ERR_INVALID_ARG, "the nonfinite word overlaps an operand");
+    }
     return CQ_OK;
 }
 
@@ -537,26 +546,36 @@ int cq_qgemv_grouped(const char* variant, const cq_gemv_problem_t* problems,
 
 int cq_int4_quantize(const void* w, void* w_packed, void* scale, int64_t n,
                      int64_t k, int scale_mode, void* stream) {
+    return cq_int4_quantize_flagged(w, w_packed, scale, n, k, scale_mode, nullptr, stream);
+}
+
+int cq_q8_quantize(const void* w, void* w_q, void* scale, int64_t n, int64_t k,
+                   int scale_mode, void* stream) {
+    return cq_q8_quantize_flagged(w, w_q, scale, n, k, scale_mode, nullptr, stream);
+}
+
+int cq_int4_quantize_flagged(const void* w, void* w_packed, void* scale, int64_t n,
+                             int64_t k, int scale_mode, uint32_t* nonfinite, void* stream) {
     g_last_error.clear();
-    int st = check_quantize(CQ_OP_INT4GEMV, w, w_packed, scale, n, k, scale_mode);
+    int st = check_quantize(CQ_OP_INT4GEMV, w, w_packed, scale, n, k, scale_mode, nonfinite);
     if (st != CQ_OK) return st;
     const cq::QuantPlan p = cq::plan_int4_quantize(n, k, w, w_packed);
     if (p.grid > INT_MAX) return fail(CQ_ERR_INVALID_ARG, "n * k too large for one launch");
     const hipError_t e = cq::launch_int4_quantize(p, w, w_packed, scale, n, k,
-                                                  scale_mode == CQ_SCALE_RCP,
+                                                  scale_mode == CQ_SCALE_RCP, nonfinite,
                                                   static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail(e, "kernel launch");
     return CQ_OK;
 }
 
-int cq_q8_quantize(const void* w, void* w_q, void* scale, int64_t n, int64_t k,
-                   int scale_mode, void* stream) {
+int cq_q8_quantize_flagged(const void* w, void* w_q, void* scale, int64_t n, int64_t k,
+                           int scale_mode, uint32_t* nonfinite, void* stream) {
     g_last_error.clear();
-    int st = check_quantize(CQ_OP_QGEMV, w, w_q, scale, n, k, scale_mode);
+    int st = check_quantize(CQ_OP_QGEMV, w, w_q, scale, n, k, scale_mode, nonfinite);
     if (st != CQ_OK) return st;
     const cq::QuantPlan p = cq::plan_q8_quantize(n, k, w, w_q);
     const hipError_t e = cq::launch_q8_quantize(p, w, w_q, scale, n, k,
-                                                scale_mode == CQ_SCALE_RCP,
+                                                scale_mode == CQ_SCALE_RCP, nonfinite,
                                                 static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail(e, "kernel launch");
     return CQ_OK;

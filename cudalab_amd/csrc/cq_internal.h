@@ -127,18 +127,20 @@ struct QuantPlan {
     bool fast = false;
     int block = 0;
     int64_t grid = 0;
-    int held = 0;   // INT8 fast kernel: 16-byte chunks per thread in registers
+    int threads = 0;   // INT8 fast kernel: threads per row
+    int held = 0;      // and 16-byte chunks per thread in registers
 };
 QuantPlan plan_int4_quantize(int64_t n, int64_t k, const void* w, const void* wp);
 QuantPlan plan_q8_quantize(int64_t n, int64_t k, const void* w, const void* wq);
 // `rcp`: scale = amax * fl(1/qmax) (torch's form on a GPU) instead of
-// amax / qmax (torch's form on the CPU).
+// amax / qmax (torch's form on the CPU).  `nonfinite` (may be null) is set to
+// 1 when w holds NaN or Inf.
 hipError_t launch_int4_quantize(const QuantPlan& p, const void* w, void* wp,
                                 void* scale, int64_t n, int64_t k, bool rcp,
-                                hipStream_t stream);
+                                uint32_t* nonfinite, hipStream_t stream);
 hipError_t launch_q8_quantize(const QuantPlan& p, const void* w, void* wq,
                               void* scale, int64_t n, int64_t k, bool rcp,
-                              hipStream_t stream);
+                              uint32_t* nonfinite, hipStream_t stream);
 
 // Plain streaming read of `bytes` (a multiple of 16) from `buf`: the
 // bandwidth ceiling of one launch reading that many bytes.

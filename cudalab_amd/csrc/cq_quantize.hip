@@ -21,16 +21,18 @@
 //
 // The outputs are bit-identical to those definitions.  Non-finite W is not
 // rejected here: a group (INT4) or row (INT8) holding NaN/Inf gets a
-// non-finite scale, and no finite input can give one (|amax| <= 65504), so a
-// caller checks the scale, not all of W.
+// non-finite scale, and no finite input can give one (|amax| <= 65504).  The
+// kernels also set *nonfinite to 1 then (if the pointer is given), so a caller
+// that must reject such W reads one word and not the scales: reading the
+// scales back took seven launches and a copy behind the quantizer (58 us for
+// the whole checked INT4 call at 4096x11008, of which the kernel is 21).
 //
 // Fast path.  Row-major W with K % 128 == 0 is a flat sequence of groups,
-// group g being elements [128 g, 128 g + 128) and scale element g.  Sixteen
-// lanes (one DPP row) take one group, 8 fp16 (16 bytes) each; a wave reads
-// 1 KiB of consecutive groups per load.  The amax is a max over fp16 bit
+// group g being elements [128 g, 128 g + 128) and scale element g.  Eight
+// lanes take one group, 16 consecutive fp16 (two 16-byte loads) each; a wave
+// reads 2 KiB of consecutive groups.  The amax is a max over fp16 bit
 // patterns with the sign cleared (for non-negative fp16 the bit-pattern
-// order is the value order), reduced across the 16 lanes with DPP row
-// rotations.
+// order is the value order), reduced across the 8 lanes with DPP.
 //
 // Quotient.  With r = v_rcp_f32(s) (at most 2 ulp from 1/s assumed, 1
 // documented) the exact product p = w * r satisfies
@@ -50,6 +52,7 @@
 // 0x88 / 0x80 per byte turns offset binary into two's complement.
 
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <cstdint>
 
 #include "cq_internal.h"
@@ -78,8 +81,11 @@ __device__ __forceinline__ uint4 load_stream(const uint4* p) {
     const u32x4 t = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
     return make_uint4(t.x, t.y, t.z, t.w);
 }
-__device__ __forceinline__ void store_stream(uint32_t* p, uint32_t v) {
-    __builtin_nontemporal_store(v, p);
+// 8 bytes at a 4-byte aligned address.
+typedef unsigned int u32x2_a4 __attribute__((ext_vector_type(2), aligned(4)));
+__device__ __forceinline__ void store_stream8_a4(uint32_t* p, uint32_t lo, uint32_t hi) {
+    const u32x2_a4 t = {lo, hi};
+    __builtin_nontemporal_store(t, reinterpret_cast<u32x2_a4*>(p));
 }
 __device__ __forceinline__ void store_stream(uint2* p, uint2 v) {
     const u32x2 t = {v.x, v.y};
@@ -127,6 +133,12 @@ __device__ __forceinline__ float h2f(uint32_t bits16) {
 
 __device__ __forceinline__ uint16_t f2h_bits(float f) {
     return __builtin_bit_cast(unsigned short, (_Float16)f);
+}
+
+// Non-finite amax: its exponent field is all ones.  Every thread that sees one
+// writes the same word.
+__device__ __forceinline__ void note_nonfinite(uint32_t amax_bits, uint32_t* flag) {
+    if (amax_bits >= 0x7C00u && flag != nullptr) *flag = 1u;
 }
 
 // Scale of a group / row from its amax: the CPU form (one correctly rounded
@@ -212,33 +224,43 @@ __device__ __forceinline__ uint2 q8_pack8(uint4 v, float s, float r) {
 }
 
 // ---------------------------------------------------------------- INT4 ---
-// Fast kernel: 16 lanes per group, kInt4Steps groups per 16-lane row,
-// 16 * kInt4Steps groups per 256-thread workgroup.  Requires w 16-byte and
-// wp 4-byte aligned.  (2 steps measured best of 1, 2, 4, 8.)
-constexpr int kInt4Steps = 2;
-constexpr int kInt4GroupsPerBlock = (kQBlock / 16) * kInt4Steps;
+// Fast kernel: 8 lanes per group, two adjacent 16-byte loads and one 8-byte
+// store each, 32 groups per 256-thread workgroup.  Requires w 16-byte and wp
+// 4-byte aligned.  Bound by memory (a copy of the same bytes with 16-byte
+// loads takes 19.8 us at 4096x11008, 8.3 at 4096^2); VALU work, about 6
+// instructions per element, runs under it.  Of the splits measured (us at
+// 4096x11008 / 4096^2 / 28672x8192): 16 lanes and two groups each, with
+// 4-byte stores, 22.3 / 10.6 / 101; 8 lanes 20.9 / 9.7 / 99; 8 lanes and two
+// groups each 22.1 / 10.5 / 101; 4 lanes with 16-byte stores 30 / 13 / 137
+// (its loads touch 64 bytes of every lane's 128).
+constexpr int kInt4GroupsPerBlock = kQBlock / 8;
+
+__device__ __forceinline__ uint32_t row8_max(uint32_t v) {
+    v = max(v, dpp_u32<0xB1>(v));    // quad_perm [1,0,3,2]
+    v = max(v, dpp_u32<0x4E>(v));    // quad_perm [2,3,0,1]
+    v = max(v, dpp_u32<0x141>(v));   // row_half_mirror: 8 lanes
+    return v;
+}
 
 __global__ __launch_bounds__(kQBlock) void int4_quantize_kernel(
         const uint4* __restrict__ w, uint32_t* __restrict__ wp,
-        uint16_t* __restrict__ scale, int64_t groups, bool rcp) {
-    const int lane16 = threadIdx.x & 15;
-    const int64_t g0 = (int64_t)blockIdx.x * kInt4GroupsPerBlock + (threadIdx.x >> 4);
+        uint16_t* __restrict__ scale, int64_t groups, bool rcp,
+        uint32_t* __restrict__ nonfinite) {
+    const int lane8 = threadIdx.x & 7;
+    const int64_t g = (int64_t)blockIdx.x * kInt4GroupsPerBlock + (threadIdx.x >> 3);
     // Out-of-range slots (the last workgroup) re-read the last group and
     // store nothing, so every load is one unconditional 16-byte load.
-    uint4 v[kInt4Steps];
-#pragma unroll
-    for (int u = 0; u < kInt4Steps; ++u) {
-        const int64_t g = min(g0 + u * (kQBlock / 16), groups - 1);
-        v[u] = load_stream(w + g * 16 + lane16);
-    }
-#pragma unroll
-    for (int u = 0; u < kInt4Steps; ++u) {
-        const int64_t g = g0 + u * (kQBlock / 16);
-        const float s = scale_of<7>(h2f(row16_max(amax_bits8(v[u]))), rcp);
-        const uint32_t packed = int4_pack8(v[u], s, quant_rcp(s));
-        if (g < groups) {
-            store_stream(wp + g * 16 + lane16, packed);
-            if (lane16 == 0) scale[g] = f2h_bits(s);
+    const uint4* src = w + min(g, groups - 1) * 16 + 2 * lane8;
+    const uint4 v0 = load_stream(src), v1 = load_stream(src + 1);
+    const uint32_t am = row8_max(max(amax_bits8(v0), amax_bits8(v1)));
+    const float s = scale_of<7>(h2f(am), rcp);
+    const float r = quant_rcp(s);
+    const uint32_t p0 = int4_pack8(v0, s, r), p1 = int4_pack8(v1, s, r);
+    if (g < groups) {
+        store_stream8_a4(wp + g * 16 + 2 * lane8, p0, p1);
+        if (lane8 == 0) {
+            scale[g] = f2h_bits(s);
+            note_nonfinite(am, nonfinite);
         }
     }
 }
@@ -247,7 +269,8 @@ __global__ __launch_bounds__(kQBlock) void int4_quantize_kernel(
 // elements per lane, the definition evaluated directly.
 __global__ __launch_bounds__(kQBlock) void int4_quantize_generic_kernel(
         const uint16_t* __restrict__ w, uint8_t* __restrict__ wp,
-        uint16_t* __restrict__ scale, int64_t groups, bool rcp) {
+        uint16_t* __restrict__ scale, int64_t groups, bool rcp,
+        uint32_t* __restrict__ nonfinite) {
     const int64_t g = (int64_t)blockIdx.x * (kQBlock / 64) + (threadIdx.x >> 6);
     if (g >= groups) return;                       // uniform over the wave
     const int lane = threadIdx.x & 63;
@@ -257,58 +280,69 @@ __global__ __launch_bounds__(kQBlock) void int4_quantize_generic_kernel(
     const uint32_t q0 = (uint32_t)quant_exact(h2f(e0), s, 7.f) & 0xFu;
     const uint32_t q1 = (uint32_t)quant_exact(h2f(e1), s, 7.f) & 0xFu;
     wp[g * 64 + lane] = (uint8_t)(q0 | (q1 << 4));
-    if (lane == 0) scale[g] = f2h_bits(s);
+    if (lane == 0) {
+        scale[g] = f2h_bits(s);
+        note_nonfinite(am, nonfinite);
+    }
 }
 
 // ---------------------------------------------------------------- INT8 ---
-// Fast kernel: one 256-thread workgroup per row, H 16-byte chunks per
-// thread held in registers between the amax and the quantize pass (rows up
-// to 256 * 8 * H elements); longer rows re-read the rest (from L2).  H is
-// the smallest instance that holds the row (fewer registers, more waves
-// per SIMD), at most kQ8MaxHeld.  Requires k % 8 == 0, w 16-byte and wq
-// 8-byte aligned.
-constexpr int kQ8MaxHeld = 8;
-
-template <int kQ8Held>
-__global__ __launch_bounds__(kQBlock) void q8_quantize_kernel(
+// Fast kernel: T threads per row (one wave, or two, four or eight), H 16-byte
+// chunks per thread held in registers between the amax and the quantize pass
+// (rows up to T * 8 * H elements); longer rows re-read the rest (from L2).
+// Every load is unconditional (threads past the row end re-read its last
+// chunk), so all H are in flight together.  Workgroups of 256 threads hold
+// 256 / T rows.  Requires k % 8 == 0, w 16-byte and wq 8-byte aligned.
+template <int T, int H>
+__global__ __launch_bounds__(T < kQBlock ? kQBlock : T) void q8_quantize_kernel(
         const uint4* __restrict__ w, uint2* __restrict__ wq,
-        float* __restrict__ scale, int64_t chunks, bool rcp) {
-    __shared__ uint32_t red[kQBlock / 64];
-    const int64_t row = blockIdx.x;
-    const uint4* src = w + row * chunks;
-    uint2* dst = wq + row * chunks;
-    uint4 v[kQ8Held];
+        float* __restrict__ scale, int64_t n, int64_t chunks, bool rcp,
+        uint32_t* __restrict__ nonfinite) {
+    constexpr int kThreads = T < kQBlock ? kQBlock : T;
+    constexpr int kRows = kThreads / T;
+    const int t = threadIdx.x % T;
+    const int64_t row = (int64_t)blockIdx.x * kRows + threadIdx.x / T;
+    const int64_t rowc = min(row, n - 1);
+    const uint4* src = w + rowc * chunks;
+    uint4 v[H];
     uint32_t am = 0;
 #pragma unroll
-    for (int h = 0; h < kQ8Held; ++h) {
-        const int64_t c = threadIdx.x + (int64_t)h * kQBlock;
-        v[h] = c < chunks ? load_stream(src + c) : make_uint4(0, 0, 0, 0);
-    }
+    for (int h = 0; h < H; ++h)
+        v[h] = load_stream(src + min((int64_t)t + h * T, chunks - 1));
 #pragma unroll
-    for (int h = 0; h < kQ8Held; ++h) am = max(am, amax_bits8(v[h]));
-    for (int64_t c = threadIdx.x + (int64_t)kQ8Held * kQBlock; c < chunks; c += kQBlock)
-        am = max(am, amax_bits8(src[c]));
+    for (int h = 0; h < H; ++h) am = max(am, amax_bits8(v[h]));
+    for (int64_t c = t + (int64_t)H * T; c < chunks; c += T) am = max(am, amax_bits8(src[c]));
     am = wave_max(am);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = am;
-    __syncthreads();
-    am = max(max(red[0], red[1]), max(red[2], red[3]));
+    if constexpr (T > 64) {
+        __shared__ uint32_t red[kThreads / 64];
+        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = am;
+        __syncthreads();
+        const int first = (threadIdx.x / T) * (T / 64);
+#pragma unroll
+        for (int i = 0; i < T / 64; ++i) am = max(am, red[first + i]);
+    }
     const float s = scale_of<127>(h2f(am), rcp);
     const float r = quant_rcp(s);
-    if (threadIdx.x == 0) scale[row] = s;
+    if (row >= n) return;
+    uint2* dst = wq + row * chunks;
+    if (t == 0) {
+        scale[row] = s;
+        note_nonfinite(am, nonfinite);
+    }
 #pragma unroll
-    for (int h = 0; h < kQ8Held; ++h) {
-        const int64_t c = threadIdx.x + (int64_t)h * kQBlock;
+    for (int h = 0; h < H; ++h) {
+        const int64_t c = t + (int64_t)h * T;
         if (c < chunks) store_stream(dst + c, q8_pack8(v[h], s, r));
     }
-    for (int64_t c = threadIdx.x + (int64_t)kQ8Held * kQBlock; c < chunks; c += kQBlock)
-        dst[c] = q8_pack8(src[c], s, r);
+    for (int64_t c = t + (int64_t)H * T; c < chunks; c += T) dst[c] = q8_pack8(src[c], s, r);
 }
 
 // Generic kernel (any k, any 2-byte aligned w): one workgroup per row,
 // element by element, the definition evaluated directly.
 __global__ __launch_bounds__(kQBlock) void q8_quantize_generic_kernel(
         const uint16_t* __restrict__ w, int8_t* __restrict__ wq,
-        float* __restrict__ scale, int64_t k, bool rcp) {
+        float* __restrict__ scale, int64_t k, bool rcp,
+        uint32_t* __restrict__ nonfinite) {
     __shared__ uint32_t red[kQBlock / 64];
     const int64_t row = blockIdx.x;
     const uint16_t* src = w + row * k;
@@ -319,7 +353,10 @@ __global__ __launch_bounds__(kQBlock) void q8_quantize_generic_kernel(
     __syncthreads();
     am = max(max(red[0], red[1]), max(red[2], red[3]));
     const float s = scale_of<127>(h2f(am), rcp);
-    if (threadIdx.x == 0) scale[row] = s;
+    if (threadIdx.x == 0) {
+        scale[row] = s;
+        note_nonfinite(am, nonfinite);
+    }
     for (int64_t i = threadIdx.x; i < k; i += kQBlock)
         wq[row * k + i] = (int8_t)quant_exact(h2f(src[i]), s, 127.f);
 }
@@ -338,52 +375,70 @@ QuantPlan plan_int4_quantize(int64_t n, int64_t k, const void* w, const void* wp
     return p;
 }
 
+// Threads per row and held chunks of the INT8 fast kernel, from the row's
+// length: as few threads as keep at most three or four chunks each.  A row
+// of few chunks wastes a workgroup, one of many waits on too many registers
+// (us per call; before, 256 threads at every length with a branch around
+// each load): 32768x1024 one wave 18.0, two 21.7, four 29.0 (before 28.1);
+// 16384x3072 two waves 25.6, four 27.5; 11008x4096 four 23.5, eight 29.3
+// (24.2); 4096x11008 eight 23.7, four 24.8, sixteen 26.8 (26.7);
+// 2048x16384 eight 19.2, sixteen 20.0 (24.3).
 QuantPlan plan_q8_quantize(int64_t n, int64_t k, const void* w, const void* wq) {
     QuantPlan p;
     p.fast = k % 8 == 0 && aligned(w, 16) && aligned(wq, 8);
     p.block = kQBlock;
     p.grid = n;
     if (p.fast) {
-        const int64_t need = (k / 8 + kQBlock - 1) / kQBlock;
-        p.held = need <= 1 ? 1 : need <= 2 ? 2 : need <= 3 ? 3 : need <= 4 ? 4
-               : need <= 6 ? 6 : kQ8MaxHeld;
+        const int64_t chunks = k / 8;
+        p.threads = chunks <= 192 ? 64 : chunks <= 384 ? 128 : chunks <= 1024 ? 256 : 512;
+        const int64_t need = (chunks + p.threads - 1) / p.threads;
+        p.held = need <= 1 ? 1 : need <= 2 ? 2 : need <= 3 ? 3 : need <= 4 ? 4 : 8;
+        p.block = std::max(kQBlock, p.threads);
+        const int64_t rows = p.block / p.threads;
+        p.grid = (n + rows - 1) / rows;
     }
     return p;
 }
 
 hipError_t launch_int4_quantize(const QuantPlan& p, const void* w, void* wp,
                                 void* scale, int64_t n, int64_t k, bool rcp,
-                                hipStream_t stream) {
+                                uint32_t* nonfinite, hipStream_t stream) {
     const int64_t groups = n * (k / 128);
     if (p.fast)
         int4_quantize_kernel<<<dim3((unsigned)p.grid), dim3(kQBlock), 0, stream>>>(
-            (const uint4*)w, (uint32_t*)wp, (uint16_t*)scale, groups, rcp);
+            (const uint4*)w, (uint32_t*)wp, (uint16_t*)scale, groups, rcp, nonfinite);
     else
         int4_quantize_generic_kernel<<<dim3((unsigned)p.grid), dim3(kQBlock), 0, stream>>>(
-            (const uint16_t*)w, (uint8_t*)wp, (uint16_t*)scale, groups, rcp);
+            (const uint16_t*)w, (uint8_t*)wp, (uint16_t*)scale, groups, rcp, nonfinite);
     return hipGetLastError();
 }
 
 hipError_t launch_q8_quantize(const QuantPlan& p, const void* w, void* wq,
                               void* scale, int64_t n, int64_t k, bool rcp,
-                              hipStream_t stream) {
+                              uint32_t* nonfinite, hipStream_t stream) {
     if (p.fast) {
-        const dim3 g((unsigned)p.grid), b(kQBlock);
+        const dim3 g((unsigned)p.grid);
         const uint4* w4 = (const uint4*)w;
         uint2* q2 = (uint2*)wq;
         float* sc = (float*)scale;
         const int64_t chunks = k / 8;
-        switch (p.held) {
-        case 1: q8_quantize_kernel<1><<<g, b, 0, stream>>>(w4, q2, sc, chunks, rcp); break;
-        case 2: q8_quantize_kernel<2><<<g, b, 0, stream>>>(w4, q2, sc, chunks, rcp); break;
-        case 3: q8_quantize_kernel<3><<<g, b, 0, stream>>>(w4, q2, sc, chunks, rcp); break;
-        case 4: q8_quantize_kernel<4><<<g, b, 0, stream>>>(w4, q2, sc, chunks, rcp); break;
-        case 6: q8_quantize_kernel<6><<<g, b, 0, stream>>>(w4, q2, sc, chunks, rcp); break;
-        default: q8_quantize_kernel<kQ8MaxHeld><<<g, b, 0, stream>>>(w4, q2, sc, chunks, rcp); break;
-        }
+        auto go = [&](auto* kernel) {
+            kernel<<<g, dim3(p.block), 0, stream>>>(w4, q2, sc, n, chunks, rcp, nonfinite);
+        };
+        if (p.threads == 64)
+            go(p.held == 1 ? &q8_quantize_kernel<64, 1> : p.held == 2 ? &q8_quantize_kernel<64, 2>
+               : &q8_quantize_kernel<64, 3>);
+        else if (p.threads == 128)
+            go(p.held == 2 ? &q8_quantize_kernel<128, 2> : &q8_quantize_kernel<128, 3>);
+        else if (p.threads == 256)
+            go(p.held <= 2 ? &q8_quantize_kernel<256, 2> : p.held == 3 ? &q8_quantize_kernel<256, 3>
+               : &q8_quantize_kernel<256, 4>);
+        else
+            go(p.held == 3 ? &q8_quantize_kernel<512, 3> : p.held == 4 ? &q8_quantize_kernel<512, 4>
+               : &q8_quantize_kernel<512, 8>);
     } else
         q8_quantize_generic_kernel<<<dim3((unsigned)p.grid), dim3(kQBlock), 0, stream>>>(
-            (const uint16_t*)w, (int8_t*)wq, (float*)scale, k, rcp);
+            (const uint16_t*)w, (int8_t*)wq, (float*)scale, k, rcp, nonfinite);
     return hipGetLastError();
 }
 

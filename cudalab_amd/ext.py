@@ -762,14 +762,27 @@ def launch_floor(grid: int, block: int, warmup: int = 200,
 
 
 # ---------------------------------------------------------------- quantizers
-def _quant_launch(fn, what: str, W: torch.Tensor, q: torch.Tensor,
-                  scale: torch.Tensor, rcp: bool) -> None:
+def _quantize(op: str, W: torch.Tensor, rcp: bool, flag: Optional[torch.Tensor]
+              ) -> tuple[torch.Tensor, torch.Tensor]:
+    """Launch the quantizer of `op` on W (N, K); `flag` a pinned int32 word
+    (set to 1 if W holds NaN/Inf) or None."""
+    N, K = W.shape
+    lib = _capi.load()
+    if op == "int4gemv":
+        fn, what = lib.cq_int4_quantize_flagged, "int4 quantize"
+        q = torch.empty((N, K // 2), dtype=torch.uint8, device=W.device)
+        scale = torch.empty((N, K // 128), dtype=torch.float16, device=W.device)
+    else:
+        fn, what = lib.cq_q8_quantize_flagged, "int8 quantize"
+        q = torch.empty((N, K), dtype=torch.int8, device=W.device)
+        scale = torch.empty((N,), dtype=torch.float32, device=W.device)
     mode = _capi.CQ_SCALE_RCP if rcp else _capi.CQ_SCALE_DIV
     st = _on_device(W.device, lambda stream: fn(
-        W.data_ptr(), q.data_ptr(), scale.data_ptr(), W.size(0), W.size(1),
-        mode, stream))
+        W.data_ptr(), q.data_ptr(), scale.data_ptr(), N, K, mode,
+        None if flag is None else flag.data_ptr(), stream))
     if st != _capi.CQ_OK:
         _fail(f"{what} failed (status {st}): {_capi.last_error()}")
+    return q, scale
 
 
 def quantize_int4(W: torch.Tensor, rcp: bool = True
@@ -781,12 +794,7 @@ def quantize_int4(W: torch.Tensor, rcp: bool = True
     non-finite scale.  `rcp`: scale32 = amax * fl(1/7), as torch computes
     `amax / 7` for a GPU tensor; otherwise amax / 7 correctly rounded, as
     torch computes it for a CPU tensor."""
-    N, K = W.shape
-    wp = torch.empty((N, K // 2), dtype=torch.uint8, device=W.device)
-    scale = torch.empty((N, K // 128), dtype=torch.float16, device=W.device)
-    _quant_launch(_capi.load().cq_int4_quantize, "int4 quantize", W, wp, scale,
-                  rcp)
-    return wp, scale
+    return _quantize("int4gemv", W, rcp, None)
 
 
 def quantize_q8(W: torch.Tensor, rcp: bool = True
@@ -796,12 +804,19 @@ def quantize_q8(W: torch.Tensor, rcp: bool = True
     float32 (N,)), asynchronous on the current stream.  A row holding
     NaN/Inf gets a non-finite scale.  `rcp` as for quantize_int4 (with
     127)."""
-    N, K = W.shape
-    wq = torch.empty((N, K), dtype=torch.int8, device=W.device)
-    scale = torch.empty((N,), dtype=torch.float32, device=W.device)
-    _quant_launch(_capi.load().cq_q8_quantize, "int8 quantize", W, wq, scale,
-                  rcp)
-    return wq, scale
+    return _quantize("qgemv", W, rcp, None)
+
+
+def quantize_finite(op: str, W: torch.Tensor, rcp: bool = True
+                    ) -> tuple[torch.Tensor, torch.Tensor, bool]:
+    """quantize_int4 / quantize_q8 and whether all of W is finite, known once
+    the call returns: the kernel sets a word of pinned host memory, and the
+    call waits for the current stream and reads it.  The word is this call's
+    own, so calls from several threads do not meet."""
+    flag = torch.zeros(1, dtype=torch.int32, device="cpu", pin_memory=True)
+    q, scale = _quantize(op, W, rcp, flag)
+    torch.cuda.current_stream(W.device).synchronize()
+    return q, scale, flag.item() == 0
 
 
 def quantize_vectorized(op: str, W: torch.Tensor, out: torch.Tensor) -> bool:

@@ -69,8 +69,7 @@ def quantize_w(W: torch.Tensor, semantics: str | None = None
     or non-finite input.
 
     A CUDA W is quantized and packed by the HIP kernel (cq_int4_quantize)
-    in one pass; its non-finite check reads the scale, which is non-finite
-    exactly where a group of W holds NaN/Inf.  An empty W launches nothing
+    in one pass, which also notes NaN/Inf (ext.quantize_finite).  An empty W launches nothing
     and gets the torch formulation's empty results.
 
     `semantics` picks how `amax / qmax` is rounded, as the reference's
@@ -82,9 +81,9 @@ def quantize_w(W: torch.Tensor, semantics: str | None = None
         raise ValueError(f"semantics must be None, 'cpu' or 'gpu', got {semantics!r}")
     if W.is_cuda and W.numel() > 0:
         _check_w(W, finite=False)
-        from .ext import quantize_int4
-        W_packed, scale = quantize_int4(W, rcp=semantics != "cpu")
-        if not bool(torch.isfinite(scale).all()):
+        from .ext import quantize_finite
+        W_packed, scale, finite = quantize_finite("int4gemv", W, rcp=semantics != "cpu")
+        if not finite:
             raise ValueError(_NONFINITE)
         return W_packed, scale
     return quantize_w_torch(W, rcp=None if semantics is None else semantics == "gpu")

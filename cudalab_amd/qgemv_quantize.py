@@ -38,9 +38,8 @@ def quantize_w(W: torch.Tensor, semantics: str | None = None
     Returns (W_q int8 (N, K), scale float32 (N,)).  Raises ValueError for
     non-2-D, non-fp16, non-contiguous or non-finite input.
 
-    A CUDA W is quantized by the HIP kernel (cq_q8_quantize) in one launch;
-    its non-finite check reads the scale, which is non-finite exactly for
-    the rows of W holding NaN/Inf.  An empty W launches nothing and gets
+    A CUDA W is quantized by the HIP kernel (cq_q8_quantize) in one launch,
+    which also notes NaN/Inf (ext.quantize_finite).  An empty W launches nothing and gets
     the torch formulation's result.
 
     `semantics` picks how `amax / qmax` is rounded, as the reference's
@@ -52,9 +51,9 @@ def quantize_w(W: torch.Tensor, semantics: str | None = None
         raise ValueError(f"semantics must be None, 'cpu' or 'gpu', got {semantics!r}")
     if W.is_cuda and W.numel() > 0:
         _check_w(W, finite=False)
-        from .ext import quantize_q8
-        W_q, scale = quantize_q8(W, rcp=semantics != "cpu")
-        if not bool(torch.isfinite(scale).all()):
+        from .ext import quantize_finite
+        W_q, scale, finite = quantize_finite("qgemv", W, rcp=semantics != "cpu")
+        if not finite:
             raise ValueError(_NONFINITE)
         return W_q, scale
     return quantize_w_torch(W, rcp=None if semantics is None else semantics == "gpu")

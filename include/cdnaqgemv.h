@@ -184,6 +184,19 @@ int cq_q8_quantize(const void* w, void* w_q, void* scale, int64_t n, int64_t k,
                    int scale_mode, void* stream);
 
 /*
+ * cq_int4_quantize / cq_q8_quantize that also report NaN/Inf: *nonfinite (a
+ * 4-byte aligned word the device can write, e.g. pinned host memory; NULL to
+ * leave it out) is set to 1 if w holds NaN or Inf and is left alone
+ * otherwise.  The caller clears it before the call and reads it once the
+ * stream has passed the launch.  No reference counterpart: its quantize_w
+ * runs isfinite over all of W.
+ */
+int cq_int4_quantize_flagged(const void* w, void* w_packed, void* scale, int64_t n,
+                             int64_t k, int scale_mode, uint32_t* nonfinite, void* stream);
+int cq_q8_quantize_flagged(const void* w, void* w_q, void* scale, int64_t n, int64_t k,
+                           int scale_mode, uint32_t* nonfinite, void* stream);
+
+/*
  * 1 if the quantizer of `op` (CQ_OP_INT4GEMV or CQ_OP_QGEMV) takes its
  * vectorized kernel for these pointers and sizes (w 16-byte aligned,
  * output 4-byte (INT4) or 8-byte (INT8) aligned, k % 8 == 0 for INT8),
