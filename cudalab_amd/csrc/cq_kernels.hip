@@ -97,20 +97,36 @@ __device__ __forceinline__ float segment_sum(float v) {
 
 // Workgroups of a launch are dealt round-robin to the 8 XCDs (workgroup i
 // runs on XCD i % 8), and each XCD has its own L2.  This returns a logical
-// block index under which every XCD owns one contiguous range of logical
-// blocks, so each XCD streams one contiguous range of weight rows and
-// writes one contiguous range of y.  It is a bijection on [0, gridDim.x)
+// block index under which every XCD takes runs of RUN consecutive logical
+// blocks, the eight XCDs one run each side by side, so that neighbouring rows
+// (their scale and y lines) stay in one L2 while all XCDs together walk
+// through one region of the weights.  What is left past the last whole set of
+// runs is split into one run per XCD.  It is a bijection on [0, gridDim.x)
 // for any grid size, so it changes which workgroup computes a row, never
 // how the row is computed (outputs are bit-identical to the identity
-// mapping).  Measured on MI355X at the bench shapes: 1-5% faster for INT4
-// and up to 16% for INT8 than the identity mapping.
-__device__ __forceinline__ uint32_t xcd_contiguous_block() {
-    constexpr uint32_t kXcds = 8;
-    const uint32_t b = blockIdx.x, g = gridDim.x;
-    const uint32_t q = g / kXcds, r = g % kXcds;
-    const uint32_t xcd = b % kXcds, idx = b / kXcds;
-    return xcd * q + (xcd < r ? xcd : r) + idx;
+// mapping).  Against one contiguous range of rows per XCD, where the eight
+// XCDs read eight far-apart regions at once (us per call, HBM-cold, runs of
+// 32): INT8 8192^2 13.5 -> 12.0, INT4 8192^2 8.1 -> 7.5, INT8 11008x4096 9.05
+// -> 8.4, INT4 32000x4096 13.3 -> 12.4, FP16 32000x4096 42.1 -> 41.1; launches
+// under 10 MB level.  Runs of 8 and 64 are up to 3% slower than 32 in places.
+// Where waves hold at most two chunks per lane, runs of 64: such a launch of
+// 512 workgroups is over in 3.4 us and 1-3% slower with runs of 32 (INT4
+// 4096^2, FP16 4096x1024).  The INT8 and FP16/FP32 K-tiled kernels keep one
+// run per XCD (INT8 4096x28672 20.7 us against 20.9, FP16 3000x65536 66.9
+// against 68.0): their waves live long enough to drift apart.
+constexpr uint32_t kXcdRun = 32;
+constexpr uint32_t kXcdAll = 1u << 24;   // one run per XCD
+// Run for waves that load `chunks` 16-byte chunks per lane in all.
+constexpr uint32_t xcd_run(int chunks) { return chunks <= 2 ? 64 : kXcdRun; }
+template <uint32_t RUN = kXcdRun>
+__device__ __forceinline__ uint32_t xcd_block(uint32_t b, uint32_t g) {
+    constexpr uint32_t kXcds = 8, kSpan = kXcds * RUN;
+    const uint32_t base = b / kSpan * kSpan, xcd = b % kXcds;
+    const uint32_t span = min(g - base, kSpan);   // or what is left
+    return base + xcd * (span / kXcds) + min(xcd, span % kXcds) + (b - base) / kXcds;
 }
+template <uint32_t RUN = kXcdRun>
+__device__ __forceinline__ uint32_t xcd_block() { return xcd_block<RUN>(blockIdx.x, gridDim.x); }
 
 // ---------------------------------------------------------------- scalar
 //
@@ -278,7 +294,7 @@ __device__ __forceinline__ void scalar_rows(
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int part = wave % SP;                // this wave's share of its rows' chunks
-    const int64_t row0 = (static_cast<int64_t>(xcd_contiguous_block()) * (kBlock / 64 / SP) +
+    const int64_t row0 = (static_cast<int64_t>(xcd_block()) * (kBlock / 64 / SP) +
                           wave / SP) * R;
     const int64_t nfull = k / E;               // whole chunks of a row
     const int64_t niter = (nfull + 63) / 64;   // 64 chunks each; this wave takes part + SP i
@@ -588,7 +604,7 @@ __global__ __launch_bounds__(kBlock) void qgemv_wave_kernel(
 // high nibble is taken in place (bits 4-7) under the fp16 exponent of 64,
 // where the mantissa step is 1/16, so ((w & 0x00F000F0) ^ 0x54805480) is
 // the fp16 pair (72+q1, 72+q5) and a packed add of -72 gives (q1, q5)
-// exactly.  Workgroups take their rows through xcd_contiguous_block(); NT
+// exactly.  Workgroups take their rows through xcd_block(); NT
 // (256 or 512 threads) is chosen by the host plan.
 //
 // Address work is kept off the VALU, which these kernels are short of (the
@@ -914,7 +930,7 @@ __global__ __launch_bounds__(NT) void int4gemv_lds_kernel(
         int nchunks) {
     extern __shared__ uint4 xs[];
     int4_lds_rows<CW, J, R, NT>(w, scale, x, y, n, nchunks,
-                                xcd_contiguous_block(), xs);
+                                xcd_block<xcd_run(J * R)>(), xs);
 }
 
 // The INT4 LDS kernel with the timeline stamps (diagnostic, cq_int4_timeline):
@@ -926,7 +942,7 @@ __global__ __launch_bounds__(NT) void int4gemv_lds_stamp_kernel(
         int nchunks, uint64_t* __restrict__ stamps) {
     extern __shared__ uint4 xs[];
     int4_lds_rows<CW, J, R, NT, true>(w, scale, x, y, n, nchunks,
-                                      xcd_contiguous_block(), xs, stamps);
+                                      xcd_block<xcd_run(J * R)>(), xs, stamps);
 }
 
 template <int CW, int J, int R, int NT>
@@ -936,7 +952,7 @@ __global__ __launch_bounds__(NT) void qgemv_lds_kernel(
         int nchunks) {
     extern __shared__ uint4 xs[];
     q8_lds_rows<CW, J, R, NT>(w, scale, x, y, n, nchunks,
-                              xcd_contiguous_block(), xs);
+                              xcd_block<xcd_run(J * R)>(), xs);
 }
 
 // K-tiled LDS kernels, for rows longer than one batch of chunks held per
@@ -965,7 +981,7 @@ __global__ __launch_bounds__(NT) void int4gemv_tiled_kernel(
     constexpr int ldsw = TC + 1;
     const int tid = threadIdx.x;
     const int col = tid & 63;
-    const int64_t row0 = (static_cast<int64_t>(xcd_contiguous_block()) * (NT >> 6) + (tid >> 6)) * R;
+    const int64_t row0 = (static_cast<int64_t>(xcd_block()) * (NT >> 6) + (tid >> 6)) * R;
     // Byte offsets within a row fit in 32 bits (the host checks
     // n * k / 2 < 2^32); row bases are 64-bit.
     const char* wrow[R];
@@ -1073,7 +1089,7 @@ __global__ __launch_bounds__(NT) void qgemv_tiled_kernel(
     constexpr int ldsw = TC + 1;
     const int tid = threadIdx.x;
     const int col = tid & 63;
-    const int64_t row0 = (static_cast<int64_t>(xcd_contiguous_block()) * (NT >> 6) + (tid >> 6)) * R;
+    const int64_t row0 = (static_cast<int64_t>(xcd_block<kXcdAll>()) * (NT >> 6) + (tid >> 6)) * R;
     const char* wrow[R];
     float sc[R];   // row scales, loaded first so the final scaling waits on nothing
 #pragma unroll
@@ -1200,7 +1216,7 @@ template <int CW, int J, int R, int NT>
 __global__ __launch_bounds__(NT) void int4gemv_lds_group_kernel(GroupArgs g,
                                                                  int nchunks) {
     extern __shared__ uint4 xs[];
-    const uint32_t lb = xcd_contiguous_block();
+    const uint32_t lb = xcd_block<xcd_run(J * R)>();
     const int p = group_of(g, lb);
     int4_lds_rows<CW, J, R, NT>(static_cast<const uint4*>(g.w[p]),
                                 static_cast<const uint16_t*>(g.scale[p]),
@@ -1213,7 +1229,7 @@ template <int CW, int J, int R, int NT>
 __global__ __launch_bounds__(NT) void qgemv_lds_group_kernel(GroupArgs g,
                                                              int nchunks) {
     extern __shared__ uint4 xs[];
-    const uint32_t lb = xcd_contiguous_block();
+    const uint32_t lb = xcd_block<xcd_run(J * R)>();
     const int p = group_of(g, lb);
     q8_lds_rows<CW, J, R, NT>(static_cast<const uint4*>(g.w[p]),
                               static_cast<const float*>(g.scale[p]),
@@ -1285,7 +1301,7 @@ __global__ __launch_bounds__(NT) void gemv_lds_kernel(
     const int lane = tid & 63;
     const int col = lane % CW;
     const int slot = lane / CW;
-    const uint32_t blk = xcd_contiguous_block();
+    const uint32_t blk = xcd_block<xcd_run(JB)>();
     const int64_t row =
         (static_cast<int64_t>(blk) * (NT >> 6) + (tid >> 6)) * SLOTS + slot;
     const uint32_t rowc = static_cast<uint32_t>(std::min<int64_t>(row, n - 1));
@@ -1367,7 +1383,7 @@ __global__ __launch_bounds__(NT) void gemv_tiled_kernel(
     static_assert(TC % NT == 0, "a tile's chunks divide over the workgroup");
     const int tid = threadIdx.x;
     const int col = tid & 63;
-    const int64_t row = static_cast<int64_t>(xcd_contiguous_block()) * (NT >> 6) + (tid >> 6);
+    const int64_t row = static_cast<int64_t>(xcd_block<kXcdAll>()) * (NT >> 6) + (tid >> 6);
     const uint64_t rowc = static_cast<uint64_t>(std::min<int64_t>(row, n - 1));
     const char* wrow = reinterpret_cast<const char*>(w) +
                        rowc * (static_cast<uint32_t>(nchunks) * 16u);
