@@ -528,11 +528,12 @@ def main(argv=None) -> int:
                                        "sets, from a HIP graph: the per-launch cost "
                                        "shared by 8 GEMVs; not the headline caliber")
         if plan.get("kernel") == "lds":
-            from cudalab_amd.evaluator.timeline import by_workgroup, run_stamped, summarize
+            from cudalab_amd.evaluator.timeline import by_workgroup, run_stamped, summarize, xcd_run
             tl = run_stamped(args.variant, sets, n_launches=400, warmup=args.warmup,
                              burn_ms=100.0)
             ts = summarize(tl["stamps"], tl["ticks_per_us"])
-            bw = by_workgroup(tl["stamps"], tl["ticks_per_us"], int(plan["block"]) // 64)
+            bw = by_workgroup(tl["stamps"], tl["ticks_per_us"], int(plan["block"]) // 64,
+                              run=xcd_run(plan))
             body_span_us = ts["span_us"]
             detail["wave_timeline"] = {
                 "span_us": round(ts["span_us"], 3),

@@ -107,22 +107,30 @@ def summarize(stamps: np.ndarray, ticks_per_us: float, skip: float = 0.25) -> di
             "launches_used": len(span)}
 
 
-def xcd_of_logical_block(grid: int) -> np.ndarray:
-    """XCD of each logical block under the kernels' XCD-contiguous mapping:
-    workgroup i runs on XCD i % 8 and each XCD owns one contiguous range of
-    logical blocks (cq_kernels.hip, xcd_contiguous_block)."""
-    q, r = divmod(grid, 8)
-    starts = [x * q + min(x, r) for x in range(9)]
+def xcd_run(plan: dict) -> int:
+    """Consecutive logical blocks an XCD takes at a time under a plan of the
+    LDS kernel (cq_kernels.hip, xcd_run)."""
+    return 64 if int(plan["j"]) * int(plan["r"]) <= 2 else 32
+
+
+def xcd_of_logical_block(grid: int, run: int = 32) -> np.ndarray:
+    """XCD of each logical block under the kernels' block mapping: workgroup
+    i runs on XCD i % 8, the XCDs take runs of `run` logical blocks side by
+    side, and what is left past the last whole set of runs is split into one
+    range per XCD (cq_kernels.hip, xcd_block)."""
     out = np.empty(grid, dtype=np.int64)
-    for x in range(8):
-        out[starts[x]:starts[x + 1]] = x
+    for base in range(0, grid, 8 * run):
+        q, r = divmod(min(grid - base, 8 * run), 8)
+        for x in range(8):
+            lo = base + x * q + min(x, r)
+            out[lo:lo + q + (x < r)] = x
     return out
 
 
 def by_workgroup(stamps: np.ndarray, ticks_per_us: float, waves_per_group: int,
-                 skip: float = 0.25) -> dict:
+                 skip: float = 0.25, run: int = 32) -> dict:
     """Per-workgroup view of the stamps (launches, waves, 8), waves in
-    logical-block order.  A workgroup's barrier time is its waves' latest
+    logical-block order, `run` the launch's xcd_run.  A workgroup's barrier time is its waves' latest
     x-barrier stamp (they all wait at one barrier), its start their earliest
     start, both from the launch's first wave start.  Workgroups of one launch
     that share a CU (their XCD and hardware CU id, stamp word 5) are ranked
@@ -138,7 +146,7 @@ def by_workgroup(stamps: np.ndarray, ticks_per_us: float, waves_per_group: int,
     rel = (t - t[:, :, 0].min(axis=1)[:, None, None]) / ticks_per_us
     start = rel[:, :, 0].reshape(-1, grid, waves_per_group).min(axis=2)
     barrier = rel[:, :, 1].reshape(-1, grid, waves_per_group).max(axis=2)
-    xcd = xcd_of_logical_block(grid)
+    xcd = xcd_of_logical_block(grid, run)
     # a CU is keyed by its XCD and its hardware CU id (the id alone need not
     # distinguish XCDs)
     cu = (stamps[lo:, :, 5].reshape(-1, grid, waves_per_group)[:, :, 0].astype(np.int64)
@@ -177,8 +185,9 @@ def run(n: int = 4096, k: int = 4096, variant: str = "int4gemv_cdna4",
     s = summarize(r["stamps"], r["ticks_per_us"])
     W0, _, x0, _ = sets[0]
     from ..ext import Int4gemvExt
-    wpg = int(Int4gemvExt().describe(variant, W0, x0)["block"]) // 64
-    s["by_workgroup"] = by_workgroup(r["stamps"], r["ticks_per_us"], wpg)
+    plan = Int4gemvExt().describe(variant, W0, x0)
+    s["by_workgroup"] = by_workgroup(r["stamps"], r["ticks_per_us"],
+                                     int(plan["block"]) // 64, run=xcd_run(plan))
     product = window_us("int4gemv", variant, sets, steps=2000, warmup=200)
     return {"variant": variant, "N": n, "K": k, "pool_sets": len(sets),
             "algorithmic_bytes": nbytes, "waves_per_launch": r["waves"],
