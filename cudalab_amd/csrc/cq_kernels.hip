@@ -618,8 +618,8 @@ __global__ __launch_bounds__(kBlock) void qgemv_wave_kernel(
 // - The row base is wave-uniform when a row spans the wave (CW = 64), so it
 //   lives in scalar registers.
 // Issue order, pinned with scheduling barriers: the workgroup's x pieces,
-// then per row, chunk by chunk, the group scale and the weight chunk
-// (INT8: the chunks, then the row scale), so that the wait before chunk j
+// then per row, chunk by chunk, the weight chunk and the group scale (the
+// grouped kernels know the weights' address before the scales'; INT8: the chunks, then the row scale), so that the wait before chunk j
 // covers chunks 0..j only and each chunk is summed as it lands.  A
 // scheduling barrier after the workgroup barrier keeps weight arithmetic
 // (and its waits) from being hoisted above it.
@@ -646,21 +646,43 @@ __device__ __forceinline__ uint64_t wall_clock_through(uint32_t& a, uint32_t& b,
     return t;
 }
 
-// The rows of logical workgroup `blk` of one INT4 problem.  `xs` is the
-// workgroup's LDS: [4][CW*J + 1] re-paired x pieces, q-major.
+// The rows a workgroup computes: logical workgroup `blk` of a problem of n
+// rows, problem `p` of its group.
+struct RowSlot {
+    int p;
+    uint32_t blk;
+    int n;
+};
+
+// Operands of a launch of one problem; the grouped kernels have their own.
+// `slot()` is evaluated behind the x loads, `scale` behind the first weight
+// load, `y` at the end: none holds back a load that does not need it.
+template <typename S, uint32_t RUN>
+struct OneProblem {
+    const uint4* w_;
+    const S* scale_;
+    uint16_t* y_;
+    int n_;
+    __device__ __forceinline__ RowSlot slot() const { return {0, xcd_block<RUN>(), n_}; }
+    __device__ __forceinline__ const uint4* w(const RowSlot&) const { return w_; }
+    __device__ __forceinline__ const S* scale(const RowSlot&) const { return scale_; }
+    __device__ __forceinline__ uint16_t* y(const RowSlot&) const { return y_; }
+};
+
+// One workgroup's rows of one INT4 problem.  `xs` is the workgroup's LDS:
+// [4][CW*J + 1] re-paired x pieces, q-major.  `ops` names the workgroup's
+// operands (OneProblem).
 //
 // STAMP (the timeline diagnostic only; every GEMV instance has it false, and
 // then none of its code exists): lane 0 of each wave writes 8 words to
 // stamps[wave * 8 ..]: the 100 MHz wall clock at the wave's start, after the
 // x barrier, after its first chunk is summed, after its last chunk is
 // summed and after its y stores are issued; then the hardware CU id.
-template <int CW, int J, int R, int NT, bool STAMP = false>
+template <int CW, int J, int R, int NT, bool STAMP = false, class Ops>
 __device__ __forceinline__ void int4_lds_rows(
-        const uint4* __restrict__ w,         // [n][nchunks] 16-byte chunks
-        const uint16_t* __restrict__ scale,  // [n][nchunks/4]
         const uint4* __restrict__ x,         // [4*nchunks] 16-byte pieces
-        uint16_t* __restrict__ y, int n, int nchunks, uint32_t blk,
-        uint4* __restrict__ xs, uint64_t* __restrict__ stamps = nullptr) {
+        int nchunks, uint4* __restrict__ xs, const Ops ops,
+        uint64_t* __restrict__ stamps = nullptr) {
     [[maybe_unused]] uint64_t ts[5] = {};
     if constexpr (STAMP) ts[0] = wall_clock64();
     constexpr int SLOTS = 64 / CW;
@@ -671,22 +693,25 @@ __device__ __forceinline__ void int4_lds_rows(
     const int col = lane % CW;
     const int slot = lane / CW;
     const int npieces = 4 * nchunks;
-    const int64_t wave_id = static_cast<int64_t>(blk) * (NT >> 6) +
-                            __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int64_t row0 = wave_id * (SLOTS * R) + slot;
-    // Byte offsets fit in 32 bits (the host checks n * k / 2 < 2^32).
-    const char* wb = reinterpret_cast<const char*>(w);
-    const char* sb = reinterpret_cast<const char*>(scale);
-    const uint32_t wrow_bytes = static_cast<uint32_t>(nchunks) * 16u;
-    const uint32_t srow_bytes = static_cast<uint32_t>(nchunks >> 2) * 2u;
 
     // (1) this thread's share of x first
     uint4 xv[XPER];
 #pragma unroll
     for (int i = 0; i < XPER; ++i) xv[i] = x[std::min(tid + i * NT, npieces - 1)];
     __builtin_amdgcn_sched_barrier(0);
-    // (2) per row, each chunk's group scale and then the chunk, all in
-    //     flight together; a last chunk past the row end re-reads chunk
+    const RowSlot g = ops.slot();
+    const int n = g.n;
+    const uint32_t blk = g.blk;
+    const int64_t wave_id = static_cast<int64_t>(blk) * (NT >> 6) +
+                            __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t row0 = wave_id * (SLOTS * R) + slot;
+    // Byte offsets fit in 32 bits (the host checks n * k / 2 < 2^32).
+    const char* wb = reinterpret_cast<const char*>(ops.w(g));
+    const char* sb = nullptr;
+    const uint32_t wrow_bytes = static_cast<uint32_t>(nchunks) * 16u;
+    const uint32_t srow_bytes = static_cast<uint32_t>(nchunks >> 2) * 2u;
+    // (2) per row, each chunk and then its group scale, all in flight
+    //     together; a last chunk past the row end re-reads chunk
     //     nchunks - 1 (x is zero there)
     const int clast = col + CW * (J - 1);
     const int cl = clast < nchunks ? clast : nchunks - 1;
@@ -698,15 +723,16 @@ __device__ __forceinline__ void int4_lds_rows(
     for (int r = 0; r < R; ++r) {
         const uint32_t row = static_cast<uint32_t>(std::min<int64_t>(row0 + SLOTS * r, n - 1));
         const char* wr = wb + row * wrow_bytes;
-        const char* sr = sb + row * srow_bytes;
 #pragma unroll
         for (int j = 0; j < J; ++j) {
             const bool in_row = j < J - 1;
-            sv[r][j] = *reinterpret_cast<const uint16_t*>(
-                sr + (in_row ? scol + (CW / 2) * j : static_cast<uint32_t>(cl >> 2) * 2u));
-            __builtin_amdgcn_sched_barrier(0);
             wv[r][j] = *reinterpret_cast<const uint4*>(
                 wr + (in_row ? wcol + CW * 16 * j : static_cast<uint32_t>(cl) * 16u));
+            __builtin_amdgcn_sched_barrier(0);
+            if (r == 0 && j == 0) sb = reinterpret_cast<const char*>(ops.scale(g));
+            const char* sr = sb + row * srow_bytes;
+            sv[r][j] = *reinterpret_cast<const uint16_t*>(
+                sr + (in_row ? scol + (CW / 2) * j : static_cast<uint32_t>(cl >> 2) * 2u));
             __builtin_amdgcn_sched_barrier(0);
         }
     }
@@ -792,7 +818,7 @@ __device__ __forceinline__ void int4_lds_rows(
         }
         acc = segment_sum<CW>(acc);
         const int64_t row = row0 + SLOTS * r;
-        if (col == CW - 1 && row < n) y[row] = f2h(acc);
+        if (col == CW - 1 && row < n) ops.y(g)[row] = f2h(acc);
     }
     if constexpr (STAMP) {
         __builtin_amdgcn_sched_barrier(0);
@@ -810,17 +836,14 @@ __device__ __forceinline__ void int4_lds_rows(
     }
 }
 
-// The rows of logical workgroup `blk` of one INT8 problem; `xs` holds
-// [2][CW*J + 1] re-paired x pieces, q-major, column CW*J zero.  Same
-// layout and issue order as the INT4 rows; the row's scale is loaded right
-// after its weights, so the final scaling waits on no load of its own.
-template <int CW, int J, int R, int NT>
+// One workgroup's rows of one INT8 problem; `xs` holds [2][CW*J + 1]
+// re-paired x pieces, q-major, column CW*J zero.  Same layout and issue order
+// as the INT4 rows; the row's scale is loaded right after its weights, so the
+// final scaling waits on no load of its own.
+template <int CW, int J, int R, int NT, class Ops>
 __device__ __forceinline__ void q8_lds_rows(
-        const uint4* __restrict__ w,       // [n][nchunks] 16 int8 per chunk
-        const float* __restrict__ scale,   // [n]
         const uint4* __restrict__ x,       // [2*nchunks] 16-byte pieces
-        uint16_t* __restrict__ y, int n, int nchunks, uint32_t blk,
-        uint4* __restrict__ xs) {
+        int nchunks, uint4* __restrict__ xs, const Ops ops) {
     constexpr int SLOTS = 64 / CW;
     constexpr int S = CW * J + 1;
     constexpr int XPER = (2 * CW * J + NT - 1) / NT;
@@ -829,16 +852,18 @@ __device__ __forceinline__ void q8_lds_rows(
     const int col = lane % CW;
     const int slot = lane / CW;
     const int npieces = 2 * nchunks;
-    const int64_t wave_id = static_cast<int64_t>(blk) * (NT >> 6) +
-                            __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int64_t row0 = wave_id * (SLOTS * R) + slot;
-    const char* wb = reinterpret_cast<const char*>(w);
-    const uint32_t wrow_bytes = static_cast<uint32_t>(nchunks) * 16u;
 
     uint4 xv[XPER];
 #pragma unroll
     for (int i = 0; i < XPER; ++i) xv[i] = x[std::min(tid + i * NT, npieces - 1)];
     __builtin_amdgcn_sched_barrier(0);
+    const RowSlot g = ops.slot();
+    const int n = g.n;
+    const int64_t wave_id = static_cast<int64_t>(g.blk) * (NT >> 6) +
+                            __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t row0 = wave_id * (SLOTS * R) + slot;
+    const char* wb = reinterpret_cast<const char*>(ops.w(g));
+    const uint32_t wrow_bytes = static_cast<uint32_t>(nchunks) * 16u;
     const int clast = col + CW * (J - 1);
     const int cl = clast < nchunks ? clast : nchunks - 1;
     const uint32_t wcol = static_cast<uint32_t>(col) * 16u;
@@ -855,7 +880,7 @@ __device__ __forceinline__ void q8_lds_rows(
             wv[r][j] = *reinterpret_cast<const uint4*>(wr + off);
             __builtin_amdgcn_sched_barrier(0);
         }
-        sc[r] = scale[row];
+        sc[r] = ops.scale(g)[row];
         __builtin_amdgcn_sched_barrier(0);
     }
     // re-pair x: piece = x0..x7 -> [(x0,x2), (x1,x3), (x4,x6), (x5,x7)]
@@ -904,7 +929,7 @@ __device__ __forceinline__ void q8_lds_rows(
         }
         acc = segment_sum<CW>(acc);
         const int64_t row = row0 + SLOTS * r;
-        if (col == CW - 1 && row < n) y[row] = f2h(sc[r] * acc);
+        if (col == CW - 1 && row < n) ops.y(g)[row] = f2h(sc[r] * acc);
     }
 }
 
@@ -929,8 +954,7 @@ __global__ __launch_bounds__(NT) void int4gemv_lds_kernel(
         const uint4* __restrict__ x, uint16_t* __restrict__ y, int n,
         int nchunks) {
     extern __shared__ uint4 xs[];
-    int4_lds_rows<CW, J, R, NT>(w, scale, x, y, n, nchunks,
-                                xcd_block<xcd_run(J * R)>(), xs);
+    int4_lds_rows<CW, J, R, NT>(x, nchunks, xs, OneProblem<uint16_t, xcd_run(J * R)>{w, scale, y, n});
 }
 
 // The INT4 LDS kernel with the timeline stamps (diagnostic, cq_int4_timeline):
@@ -941,8 +965,8 @@ __global__ __launch_bounds__(NT) void int4gemv_lds_stamp_kernel(
         const uint4* __restrict__ x, uint16_t* __restrict__ y, int n,
         int nchunks, uint64_t* __restrict__ stamps) {
     extern __shared__ uint4 xs[];
-    int4_lds_rows<CW, J, R, NT, true>(w, scale, x, y, n, nchunks,
-                                      xcd_block<xcd_run(J * R)>(), xs, stamps);
+    int4_lds_rows<CW, J, R, NT, true>(x, nchunks, xs,
+                                      OneProblem<uint16_t, xcd_run(J * R)>{w, scale, y, n}, stamps);
 }
 
 template <int CW, int J, int R, int NT>
@@ -951,8 +975,7 @@ __global__ __launch_bounds__(NT) void qgemv_lds_kernel(
         const uint4* __restrict__ x, uint16_t* __restrict__ y, int n,
         int nchunks) {
     extern __shared__ uint4 xs[];
-    q8_lds_rows<CW, J, R, NT>(w, scale, x, y, n, nchunks,
-                              xcd_block<xcd_run(J * R)>(), xs);
+    q8_lds_rows<CW, J, R, NT>(x, nchunks, xs, OneProblem<float, xcd_run(J * R)>{w, scale, y, n});
 }
 
 // K-tiled LDS kernels, for rows longer than one batch of chunks held per
@@ -1190,54 +1213,149 @@ constexpr uint32_t tile_lds(int pieces, int tj) {
     return static_cast<uint32_t>(pieces) * (tj * 64 + 1) * 16u;
 }
 
-// Several independent problems of one k per launch (grouped GEMV).  The
-// problem table travels by value in the kernel arguments; logical
+// Several independent problems of one k per launch (grouped GEMV).  Logical
 // workgroups [start[p], start[p+1]) belong to problem p, and each computes
 // exactly the rows it would compute in a launch of that problem alone, so
 // the outputs are bit-identical to separate launches.
-struct GroupArgs {
-    const void* w[kMaxGroup];
-    const void* scale[kMaxGroup];
-    const void* x[kMaxGroup];
-    void* y[kMaxGroup];
-    int n[kMaxGroup];
-    uint32_t start[kMaxGroup + 1];
-    int count;
+//
+// What a workgroup needs before its first load travels in the kernel
+// arguments that the hardware preloads into scalar registers (the first 14
+// words), and the prefix sums of the workgroup counts are computed from the
+// row counts: a workgroup that first has to read a table from the argument
+// memory stands still for each dependent read (the table form
+// before cost 0.7-1.2 us a launch: four dependent reads):
+// - Group3 (two or three problems with one x: q/k/v, gate/up): x, the weights
+//   and the row counts are preloaded; scale and y are read behind the first
+//   weight loads.
+// - Group8 (any other group): the row counts are preloaded; one 32-byte read
+//   brings the problem's pointers.
+// INT4 us per call, before and now (problems with one x): 3 x 4096x4096
+// 7.6 -> 6.4 (one matrix of the same rows 6.3), 2 x 11008x4096 10.9 -> 9.7,
+// 1024 + 256 + 256 x 1024 3.17 -> 2.22; with an x each: 3 x 4096x4096 6.7,
+// 1024 + 256 + 256 x 1024 2.54.
+constexpr int log2_of(int v) { return v <= 1 ? 0 : 1 + log2_of(v / 2); }
+
+// Selects of values: written on the arguments themselves, they would select
+// among the arguments' addresses and put the arguments into scratch memory
+// (a grouped launch then takes twice as long).
+template <typename T>
+__device__ __forceinline__ T pick2(bool second, T a, T b) { return second ? b : a; }
+template <typename T>
+__device__ __forceinline__ T pick3(int p, T a, T b, T c) {
+    return pick2(p == 2, pick2(p == 1, a, b), c);
+}
+
+template <int ROWS, uint32_t RUN, int COUNT>   // rows per workgroup, run of xcd_block
+__device__ __forceinline__ RowSlot group_slot(const int (&n)[COUNT]) {
+    constexpr int kShift = log2_of(ROWS);
+    static_assert(ROWS == 1 << kShift, "rows per workgroup are a power of two");
+    uint32_t start[COUNT + 1] = {0};
+#pragma unroll
+    for (int i = 0; i < COUNT; ++i)
+        start[i + 1] = start[i] + ((static_cast<uint32_t>(n[i]) + ROWS - 1) >> kShift);
+    const uint32_t lb = xcd_block<RUN>(blockIdx.x, start[COUNT]);
+    RowSlot s{0, lb, n[0]};
+#pragma unroll
+    for (int i = 1; i < COUNT; ++i) {
+        const bool past = lb >= start[i];       // absent problems have no workgroups
+        s.p = pick2(past, s.p, i);
+        s.blk = pick2(past, s.blk, lb - start[i]);
+        s.n = pick2(past, s.n, n[i]);
+    }
+    return s;
+}
+
+// Two or three problems with one x.
+template <typename S, int ROWS, uint32_t RUN>
+struct Group3 {
+    const uint4* w_[3];
+    const S* scale_[3];
+    uint16_t* y_[3];
+    int n_[3];
+    __device__ __forceinline__ RowSlot slot() const { return group_slot<ROWS, RUN>(n_); }
+    __device__ __forceinline__ const uint4* w(const RowSlot& s) const {
+        return pick3(s.p, w_[0], w_[1], w_[2]);
+    }
+    __device__ __forceinline__ const S* scale(const RowSlot& s) const {
+        return pick3(s.p, scale_[0], scale_[1], scale_[2]);
+    }
+    __device__ __forceinline__ uint16_t* y(const RowSlot& s) const {
+        return pick3(s.p, y_[0], y_[1], y_[2]);
+    }
 };
 
-__device__ __forceinline__ int group_of(const GroupArgs& g, uint32_t lb) {
-    int p = 0;
-#pragma unroll
-    for (int i = 1; i < kMaxGroup; ++i) p += (i < g.count && lb >= g.start[i]) ? 1 : 0;
-    return p;
+// A problem of a larger group, its slot known before x.
+template <typename S>
+struct OneSlot {
+    const uint4* w_;
+    const S* scale_;
+    uint16_t* y_;
+    RowSlot s_;
+    __device__ __forceinline__ RowSlot slot() const { return s_; }
+    __device__ __forceinline__ const uint4* w(const RowSlot&) const { return w_; }
+    __device__ __forceinline__ const S* scale(const RowSlot&) const { return scale_; }
+    __device__ __forceinline__ uint16_t* y(const RowSlot&) const { return y_; }
+};
+
+struct GroupRecord {
+    const void* w;
+    const void* scale;
+    const void* x;
+    void* y;
+};
+struct Group8Records {
+    GroupRecord r[kMaxGroup];
+};
+
+template <int CW, int J, int R, int NT>
+__global__ __launch_bounds__(NT) void int4gemv_lds_group3_kernel(
+        const uint4* x, const uint4* w0, const uint4* w1, const uint4* w2, int n0,
+        int n1, int n2, int nchunks, const uint16_t* s0, const uint16_t* s1, const uint16_t* s2,
+        uint16_t* y0, uint16_t* y1, uint16_t* y2) {
+    extern __shared__ uint4 xs[];
+    constexpr int kRows = 64 / CW * R * (NT / 64);
+    int4_lds_rows<CW, J, R, NT>(x, nchunks, xs,
+        Group3<uint16_t, kRows, xcd_run(J * R)>{{w0, w1, w2}, {s0, s1, s2}, {y0, y1, y2},
+                                          {n0, n1, n2}});
 }
 
 template <int CW, int J, int R, int NT>
-__global__ __launch_bounds__(NT) void int4gemv_lds_group_kernel(GroupArgs g,
-                                                                 int nchunks) {
+__global__ __launch_bounds__(NT) void int4gemv_lds_group8_kernel(
+        int n0, int n1, int n2, int n3, int n4, int n5, int n6, int n7, int nchunks,
+        Group8Records g) {
     extern __shared__ uint4 xs[];
-    const uint32_t lb = xcd_block<xcd_run(J * R)>();
-    const int p = group_of(g, lb);
-    int4_lds_rows<CW, J, R, NT>(static_cast<const uint4*>(g.w[p]),
-                                static_cast<const uint16_t*>(g.scale[p]),
-                                static_cast<const uint4*>(g.x[p]),
-                                static_cast<uint16_t*>(g.y[p]), g.n[p], nchunks,
-                                lb - g.start[p], xs);
+    const int n[kMaxGroup] = {n0, n1, n2, n3, n4, n5, n6, n7};
+    const RowSlot s = group_slot<64 / CW * R * (NT / 64), xcd_run(J * R)>(n);
+    const GroupRecord r = g.r[s.p];
+    int4_lds_rows<CW, J, R, NT>(static_cast<const uint4*>(r.x), nchunks, xs,
+        OneSlot<uint16_t>{static_cast<const uint4*>(r.w), static_cast<const uint16_t*>(r.scale),
+                    static_cast<uint16_t*>(r.y), s});
 }
 
 template <int CW, int J, int R, int NT>
-__global__ __launch_bounds__(NT) void qgemv_lds_group_kernel(GroupArgs g,
-                                                             int nchunks) {
+__global__ __launch_bounds__(NT) void qgemv_lds_group3_kernel(
+        const uint4* x, const uint4* w0, const uint4* w1, const uint4* w2, int n0,
+        int n1, int n2, int nchunks, const float* s0, const float* s1, const float* s2,
+        uint16_t* y0, uint16_t* y1, uint16_t* y2) {
     extern __shared__ uint4 xs[];
-    const uint32_t lb = xcd_block<xcd_run(J * R)>();
-    const int p = group_of(g, lb);
-    q8_lds_rows<CW, J, R, NT>(static_cast<const uint4*>(g.w[p]),
-                              static_cast<const float*>(g.scale[p]),
-                              static_cast<const uint4*>(g.x[p]),
-                              static_cast<uint16_t*>(g.y[p]), g.n[p], nchunks,
-                              lb - g.start[p], xs);
+    constexpr int kRows = 64 / CW * R * (NT / 64);
+    q8_lds_rows<CW, J, R, NT>(x, nchunks, xs,
+        Group3<float, kRows, xcd_run(J * R)>{{w0, w1, w2}, {s0, s1, s2}, {y0, y1, y2},
+                                          {n0, n1, n2}});
 }
 
+template <int CW, int J, int R, int NT>
+__global__ __launch_bounds__(NT) void qgemv_lds_group8_kernel(
+        int n0, int n1, int n2, int n3, int n4, int n5, int n6, int n7, int nchunks,
+        Group8Records g) {
+    extern __shared__ uint4 xs[];
+    const int n[kMaxGroup] = {n0, n1, n2, n3, n4, n5, n6, n7};
+    const RowSlot s = group_slot<64 / CW * R * (NT / 64), xcd_run(J * R)>(n);
+    const GroupRecord r = g.r[s.p];
+    q8_lds_rows<CW, J, R, NT>(static_cast<const uint4*>(r.x), nchunks, xs,
+        OneSlot<float>{static_cast<const uint4*>(r.w), static_cast<const float*>(r.scale),
+                    static_cast<uint16_t*>(r.y), s});
+}
 
 // ------------------------------------------------------------- FP16/FP32
 //
@@ -1548,26 +1666,49 @@ struct Int4LdsStamp {
     }
 };
 
-using Int4GroupFn = void (*)(GroupArgs, int);
-using Q8GroupFn = void (*)(GroupArgs, int);
+template <typename S>
+using Group3Fn = void (*)(const uint4*, const uint4*, const uint4*, const uint4*, int,
+                          int, int, int, const S*, const S*, const S*, uint16_t*,
+                          uint16_t*, uint16_t*);
+using Group8Fn = void (*)(int, int, int, int, int, int, int, int, int, Group8Records);
 
 template <int NT>
-struct Int4LdsGroup {
-    using Fn = Int4GroupFn;
+struct Int4LdsGroup3 {
+    using Fn = Group3Fn<uint16_t>;
     static constexpr int kMaxJ = kInt4MaxJ;
     template <int CW, int J, int R>
     static constexpr Fn get() {
-        if constexpr (R <= int4_rmax(J)) return &int4gemv_lds_group_kernel<CW, J, R, NT>;
+        if constexpr (R <= int4_rmax(J)) return &int4gemv_lds_group3_kernel<CW, J, R, NT>;
         else return nullptr;
     }
 };
 template <int NT>
-struct Q8LdsGroup {
-    using Fn = Q8GroupFn;
+struct Int4LdsGroup8 {
+    using Fn = Group8Fn;
+    static constexpr int kMaxJ = kInt4MaxJ;
+    template <int CW, int J, int R>
+    static constexpr Fn get() {
+        if constexpr (R <= int4_rmax(J)) return &int4gemv_lds_group8_kernel<CW, J, R, NT>;
+        else return nullptr;
+    }
+};
+template <int NT>
+struct Q8LdsGroup3 {
+    using Fn = Group3Fn<float>;
     static constexpr int kMaxJ = kQ8MaxJ;
     template <int CW, int J, int R>
     static constexpr Fn get() {
-        if constexpr (R <= q8_rmax(J)) return &qgemv_lds_group_kernel<CW, J, R, NT>;
+        if constexpr (R <= q8_rmax(J)) return &qgemv_lds_group3_kernel<CW, J, R, NT>;
+        else return nullptr;
+    }
+};
+template <int NT>
+struct Q8LdsGroup8 {
+    using Fn = Group8Fn;
+    static constexpr int kMaxJ = kQ8MaxJ;
+    template <int CW, int J, int R>
+    static constexpr Fn get() {
+        if constexpr (R <= q8_rmax(J)) return &qgemv_lds_group8_kernel<CW, J, R, NT>;
         else return nullptr;
     }
 };
@@ -1961,46 +2102,41 @@ Plan group_plan(PlanFn plan_one, OkFn lds_ok, int rows,
     return p;
 }
 
-// Per-problem workgroup counts of plan `p` and their prefix sums.
-bool fill_group(const Plan& p, const GroupProblem* probs, int count,
-                GroupArgs& g, int64_t& grid) {
-    const int64_t rows_per_wave = static_cast<int64_t>(64 / p.cw) * p.r;
-    const int64_t block_waves = p.block / 64;
-    int64_t start = 0;
-    for (int i = 0; i < kMaxGroup; ++i) {
-        g.w[i] = g.scale[i] = g.x[i] = nullptr;
-        g.y[i] = nullptr;
-        g.n[i] = 0;
-    }
+// One grouped launch of plan `p`: the kernel for two or three problems that
+// share x, or the general one.  An absent problem has no rows.
+template <typename S>
+hipError_t launch_group(Group3Fn<S> fn3, Group8Fn fn8, const Plan& p,
+                        const GroupProblem* probs, int count, uint32_t shmem,
+                        int nchunks, hipStream_t stream) {
+    if (fn3 == nullptr || fn8 == nullptr) return hipErrorInvalidConfiguration;
+    const int64_t rows = static_cast<int64_t>(64 / p.cw) * p.r * (p.block / 64);
+    int64_t grid = 0;
+    int n[kMaxGroup] = {};
+    bool one_x = true;
     for (int i = 0; i < count; ++i) {
-        const int64_t waves = (probs[i].n + rows_per_wave - 1) / rows_per_wave;
-        g.w[i] = probs[i].w;
-        g.scale[i] = probs[i].scale;
-        g.x[i] = probs[i].x;
-        g.y[i] = probs[i].y;
-        g.n[i] = static_cast<int>(probs[i].n);
-        g.start[i] = static_cast<uint32_t>(start);
-        start += (waves + block_waves - 1) / block_waves;
-        if (start > INT32_MAX) return false;
+        n[i] = static_cast<int>(probs[i].n);
+        grid += (probs[i].n + rows - 1) / rows;
+        one_x = one_x && probs[i].x == probs[0].x;
     }
-    for (int i = count; i <= kMaxGroup; ++i) g.start[i] = static_cast<uint32_t>(start);
-    g.count = count;
-    grid = start;
-    return true;
-}
-
-template <typename Fn>
-hipError_t launch_group(Fn fn, const Plan& p, const GroupArgs& g,
-                        int64_t grid, uint32_t shmem, int nchunks,
-                        hipStream_t stream) {
-    if (fn == nullptr) return hipErrorInvalidConfiguration;
-    GroupArgs a = g;
-    int nc = nchunks;
-    void* argv[] = {static_cast<void*>(&a), static_cast<void*>(&nc)};
-    return hipLaunchKernel(reinterpret_cast<const void*>(fn),
-                           dim3(static_cast<uint32_t>(grid)),
-                           dim3(static_cast<uint32_t>(p.block)), argv, shmem,
-                           stream);
+    if (grid > INT32_MAX) return hipErrorInvalidConfiguration;
+    if (count <= 3 && one_x) {
+        const uint4* w[3] = {};
+        const S* sc[3] = {};
+        uint16_t* y[3] = {};
+        for (int i = 0; i < count; ++i) {
+            w[i] = static_cast<const uint4*>(probs[i].w);
+            sc[i] = static_cast<const S*>(probs[i].scale);
+            y[i] = static_cast<uint16_t*>(probs[i].y);
+        }
+        return launch(fn3, grid, p.block, shmem, stream, nullptr, nullptr,
+                      static_cast<const uint4*>(probs[0].x), w[0], w[1], w[2], n[0], n[1],
+                      n[2], nchunks, sc[0], sc[1], sc[2], y[0], y[1], y[2]);
+    }
+    Group8Records g = {};
+    for (int i = 0; i < count; ++i)
+        g.r[i] = {probs[i].w, probs[i].scale, probs[i].x, probs[i].y};
+    return launch(fn8, grid, p.block, shmem, stream, nullptr, nullptr, n[0], n[1], n[2],
+                  n[3], n[4], n[5], n[6], n[7], nchunks, g);
 }
 
 }  // namespace
@@ -2027,31 +2163,27 @@ Plan plan_q8_group(int rows, const GroupProblem* probs, int count, int64_t k) {
 
 hipError_t launch_int4_group(const Plan& p, const GroupProblem* probs,
                              int count, int64_t k, hipStream_t stream) {
-    if (p.kind != kLds || count < 1 || count > kMaxGroup)
+    if (p.kind != kLds || count < 1 || count > kMaxGroup || !lds_chunks_ok(p, k / 32))
         return hipErrorInvalidConfiguration;
-    GroupArgs g;
-    int64_t grid = 0;
-    if (!fill_group(p, probs, count, g, grid)) return hipErrorInvalidConfiguration;
-    const Int4GroupFn fn = p.block == 512
-                               ? instance<Int4LdsGroup<512>>(p.cw, p.j, p.r)
-                               : instance<Int4LdsGroup<kBlock>>(p.cw, p.j, p.r);
-    if (!lds_chunks_ok(p, k / 32)) return hipErrorInvalidConfiguration;
-    return launch_group(fn, p, g, grid, int4_lds_bytes(p.cw, p.j),
+    const bool wide = p.block == 512;
+    return launch_group(wide ? instance<Int4LdsGroup3<512>>(p.cw, p.j, p.r)
+                             : instance<Int4LdsGroup3<kBlock>>(p.cw, p.j, p.r),
+                        wide ? instance<Int4LdsGroup8<512>>(p.cw, p.j, p.r)
+                             : instance<Int4LdsGroup8<kBlock>>(p.cw, p.j, p.r),
+                        p, probs, count, int4_lds_bytes(p.cw, p.j),
                         static_cast<int>(k / 32), stream);
 }
 
 hipError_t launch_q8_group(const Plan& p, const GroupProblem* probs,
-                           int count, int64_t k, hipStream_t stream) {
-    if (p.kind != kLds || count < 1 || count > kMaxGroup)
+                             int count, int64_t k, hipStream_t stream) {
+    if (p.kind != kLds || count < 1 || count > kMaxGroup || !lds_chunks_ok(p, k / 16))
         return hipErrorInvalidConfiguration;
-    GroupArgs g;
-    int64_t grid = 0;
-    if (!fill_group(p, probs, count, g, grid)) return hipErrorInvalidConfiguration;
-    const Q8GroupFn fn = p.block == 512
-                             ? instance<Q8LdsGroup<512>>(p.cw, p.j, p.r)
-                             : instance<Q8LdsGroup<kBlock>>(p.cw, p.j, p.r);
-    if (!lds_chunks_ok(p, k / 16)) return hipErrorInvalidConfiguration;
-    return launch_group(fn, p, g, grid, q8_lds_bytes(p.cw, p.j),
+    const bool wide = p.block == 512;
+    return launch_group(wide ? instance<Q8LdsGroup3<512>>(p.cw, p.j, p.r)
+                             : instance<Q8LdsGroup3<kBlock>>(p.cw, p.j, p.r),
+                        wide ? instance<Q8LdsGroup8<512>>(p.cw, p.j, p.r)
+                             : instance<Q8LdsGroup8<kBlock>>(p.cw, p.j, p.r),
+                        p, probs, count, q8_lds_bytes(p.cw, p.j),
                         static_cast<int>(k / 16), stream);
 }
 
