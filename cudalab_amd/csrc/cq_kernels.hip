@@ -139,8 +139,9 @@ __device__ __forceinline__ uint32_t xcd_block() { return xcd_block<RUN>(blockIdx
 // weight chunks lane + 64 (i + SP j) of a row (E elements each) and loads x
 // for them straight from memory (every wave reads x, so it sits in the
 // caches), once for its R rows.  Batches of U chunks run through two register
-// sets: batch b + 1 is in flight while batch b is summed.  The k % E elements
-// past the last whole chunk go one per lane.  Four accumulators per lane keep
+// sets: batch b + 1 is in flight while batch b is summed (its loads are
+// unconditional, see gemv_lds_kernel).  The k % E elements past the last whole
+// chunk go one per lane.  Four accumulators per lane keep
 // the FMA chains as short as one element per thread of a 256-thread workgroup
 // would; the shares of a row meet in LDS and are added in wave order.  Chunks
 // past the row end are re-read in bounds and not summed (no zero operand
@@ -148,7 +149,7 @@ __device__ __forceinline__ uint32_t xcd_block() { return xcd_block<RUN>(blockIdx
 //
 // Bound by memory.  With one element per load and one workgroup per row (the
 // form before) the memory system was idle: INT8 4001x4099 (16 MB) 12.2 us,
-// now 6.3; FP16 4096^2 off alignment 18.3 us, now 8.0.  What is left of the
+// now 6.1; FP16 4096^2 off alignment 18.3 us, now 7.5.  What is left of the
 // distance to the aligned kernels (INT8 4096^2 4.4 us) is the loads that
 // start off a 4-byte boundary: the same INT8 4096^2 call on this kernel is
 // 5.3 us with W 4 or 8 bytes off, 6.0 with W 1 or 2 bytes off.
@@ -166,12 +167,12 @@ __device__ __forceinline__ float times_scale(_Float16 q, float s) {
 }
 
 // Per operator: E elements per 16-byte chunk, XP 16-byte pieces of x per
-// chunk, `Scale` what a chunk needs to be summed, `sum` one chunk into the
-// four accumulators, `one` a single element.
+// chunk, `sum` one chunk into the four accumulators, `one` a single element.
 struct AnyInt4 {
     using Y = uint16_t;
     static constexpr int E = 32, XP = 4, kXBytes = 2;
     static constexpr bool kGroupScale = true;
+    static constexpr bool kTailFirst = false;
     static __device__ __forceinline__ float scale_of(const void* s, int64_t, int64_t i) {
         return h2f(static_cast<const uint16_t*>(s)[i]);
     }
@@ -201,8 +202,9 @@ struct AnyInt4 {
         }
     }
     // k % 128 == 0: no element past the last whole chunk
-    static __device__ __forceinline__ float one(const char*, const char*, int64_t, float,
-                                                float acc) { return acc; }
+    static __device__ __forceinline__ float elem_w(const char*, int64_t) { return 0.f; }
+    static __device__ __forceinline__ float elem_x(const char*, int64_t) { return 0.f; }
+    static __device__ __forceinline__ float one(float, float, float, float acc) { return acc; }
     static __device__ __forceinline__ void store(Y* y, float v) { *y = f2h(v); }
 };
 
@@ -210,6 +212,7 @@ struct AnyInt8 {
     using Y = uint16_t;
     static constexpr int E = 16, XP = 2, kXBytes = 2;
     static constexpr bool kGroupScale = false;
+    static constexpr bool kTailFirst = false;
     static __device__ __forceinline__ float scale_of(const void* s, int64_t row, int64_t) {
         return static_cast<const float*>(s)[row];
     }
@@ -231,10 +234,14 @@ struct AnyInt8 {
             acc[3] = __builtin_fmaf(times_scale(qb[1], s), static_cast<float>(x23[1]), acc[3]);
         }
     }
-    static __device__ __forceinline__ float one(const char* w, const char* x, int64_t i,
-                                                float s, float acc) {
-        const float q = static_cast<float>(reinterpret_cast<const int8_t*>(w)[i]);
-        return __builtin_fmaf(q * s, h2f(reinterpret_cast<const uint16_t*>(x)[i]), acc);
+    static __device__ __forceinline__ float elem_w(const char* w, int64_t i) {
+        return static_cast<float>(reinterpret_cast<const int8_t*>(w)[i]);
+    }
+    static __device__ __forceinline__ float elem_x(const char* x, int64_t i) {
+        return h2f(reinterpret_cast<const uint16_t*>(x)[i]);
+    }
+    static __device__ __forceinline__ float one(float w, float x, float s, float acc) {
+        return __builtin_fmaf(w * s, x, acc);
     }
     static __device__ __forceinline__ void store(Y* y, float v) { *y = f2h(v); }
 };
@@ -243,6 +250,7 @@ struct AnyF16 {
     using Y = uint16_t;
     static constexpr int E = 8, XP = 1, kXBytes = 2;
     static constexpr bool kGroupScale = false;
+    static constexpr bool kTailFirst = true;
     static __device__ __forceinline__ float scale_of(const void*, int64_t, int64_t) { return 0.f; }
     static __device__ __forceinline__ void sum(const uint4& w, const uint4 (&x)[XP], float,
                                                float (&acc)[4]) {
@@ -254,10 +262,12 @@ struct AnyF16 {
             acc[i] = __builtin_fmaf(static_cast<float>(a[1]), static_cast<float>(b[1]), acc[i]);
         }
     }
-    static __device__ __forceinline__ float one(const char* w, const char* x, int64_t i, float,
-                                                float acc) {
-        return __builtin_fmaf(h2f(reinterpret_cast<const uint16_t*>(w)[i]),
-                              h2f(reinterpret_cast<const uint16_t*>(x)[i]), acc);
+    static __device__ __forceinline__ float elem_w(const char* w, int64_t i) {
+        return h2f(reinterpret_cast<const uint16_t*>(w)[i]);
+    }
+    static __device__ __forceinline__ float elem_x(const char* x, int64_t i) { return elem_w(x, i); }
+    static __device__ __forceinline__ float one(float w, float x, float, float acc) {
+        return __builtin_fmaf(w, x, acc);
     }
     static __device__ __forceinline__ void store(Y* y, float v) { *y = f2h(v); }
 };
@@ -266,6 +276,7 @@ struct AnyF32 {
     using Y = float;
     static constexpr int E = 4, XP = 1, kXBytes = 4;
     static constexpr bool kGroupScale = false;
+    static constexpr bool kTailFirst = true;
     static __device__ __forceinline__ float scale_of(const void*, int64_t, int64_t) { return 0.f; }
     static __device__ __forceinline__ void sum(const uint4& w, const uint4 (&x)[XP], float,
                                                float (&acc)[4]) {
@@ -275,10 +286,12 @@ struct AnyF32 {
             acc[i] = __builtin_fmaf(__builtin_bit_cast(float, ws[i]),
                                     __builtin_bit_cast(float, xw[i]), acc[i]);
     }
-    static __device__ __forceinline__ float one(const char* w, const char* x, int64_t i, float,
-                                                float acc) {
-        return __builtin_fmaf(reinterpret_cast<const float*>(w)[i],
-                              reinterpret_cast<const float*>(x)[i], acc);
+    static __device__ __forceinline__ float elem_w(const char* w, int64_t i) {
+        return reinterpret_cast<const float*>(w)[i];
+    }
+    static __device__ __forceinline__ float elem_x(const char* x, int64_t i) { return elem_w(x, i); }
+    static __device__ __forceinline__ float one(float w, float x, float, float acc) {
+        return __builtin_fmaf(w, x, acc);
     }
     static __device__ __forceinline__ void store(Y* y, float v) { *y = v; }
 };
@@ -332,7 +345,21 @@ __device__ __forceinline__ void scalar_rows(
 #pragma unroll
             for (int p = 0; p < XP; ++p) b.x[u][p] = load16_any(xp + 16 * p);
         }
+        __builtin_amdgcn_sched_barrier(0);
     };
+    // The elements past the last whole chunk, one per lane, in the last wave;
+    // loaded ahead of the chunks where those are few elements each (FP16
+    // 32000x2050 20.8 us against 22.6, FP32 20000x1001 13.4 against 15.2), at
+    // the end for INT8 (4001x4099 6.1 against 6.2, 16001x4099 16.8 against 17.5).
+    const int64_t tail = nfull * E + lane;
+    const int64_t tail_in = std::min<int64_t>(tail, k - 1);
+    float tail_w[R] = {}, tail_x = 0.f;
+    auto load_tail = [&] {
+        tail_x = Op::elem_x(x, tail_in);
+#pragma unroll
+        for (int r = 0; r < R; ++r) tail_w[r] = Op::elem_w(wr[r], tail_in);
+    };
+    if constexpr (Op::kTailFirst) load_tail();
     float acc[R][4] = {};
     auto sum = [&](const Batch& b, int64_t it0) {
 #pragma unroll
@@ -345,20 +372,26 @@ __device__ __forceinline__ void scalar_rows(
         constexpr int64_t kStep = SP * U;
         Batch b0, b1;
         load(b0, part);
-        for (int64_t it = part; it < niter; it += 2 * kStep) {
-            if (it + kStep < niter) load(b1, it + kStep);
+        int64_t it = part;
+        for (; it + 2 * kStep < niter; it += 2 * kStep) {
+            load(b1, it + kStep);
             sum(b0, it);
-            if (it + kStep < niter) {
-                if (it + 2 * kStep < niter) load(b0, it + 2 * kStep);
-                sum(b1, it + kStep);
-            }
+            load(b0, it + 2 * kStep);
+            sum(b1, it + kStep);
+        }
+        if (it + kStep < niter) {
+            load(b1, it + kStep);
+            sum(b0, it);
+            sum(b1, it + kStep);
+        } else {
+            sum(b0, it);
         }
     }
-    // the elements past the last whole chunk, one per lane, by the last wave
-    const int64_t tail = nfull * E + lane;
-    if (part == SP - 1 && tail < k)
+    if (part == SP - 1 && tail < k) {
+        if constexpr (!Op::kTailFirst) load_tail();
 #pragma unroll
-        for (int r = 0; r < R; ++r) acc[r][0] = Op::one(wr[r], x, tail, srow[r], acc[r][0]);
+        for (int r = 0; r < R; ++r) acc[r][0] = Op::one(tail_w[r], tail_x, srow[r], acc[r][0]);
+    }
     float a[R];
 #pragma unroll
     for (int r = 0; r < R; ++r)
@@ -1401,7 +1434,13 @@ __device__ __forceinline__ void dot_chunk(float, const uint4& w,
 // ([nchunks + 1] chunks, the last one zero: what lanes past the row end
 // read).  The lane's W chunks stream through two register batches of JB
 // chunks: batch b+1 is in flight while batch b is multiplied, so any K
-// runs with a bounded register budget.
+// runs with a bounded register budget.  The loop's loads are unconditional (the
+// last batch is peeled): after a load under a condition the compiler no longer
+// knows how many are in flight and waits for all of them before it multiplies.
+// FP16 4096x11008 17.5 -> 16.8 us, 1000x30000 16.6 -> 15.7, 32000x4096 41.1 ->
+// 40.3, FP32 2000x14000 23.7 -> 22.9.  (The K-tiled kernel below keeps its
+// conditional loads: four batches a tile between two barriers gain nothing,
+// 3000x65536 67.2 us against 66.6.)
 constexpr int kGemvBatch = 8;
 
 // JB: chunks per lane per register batch, the smaller of kGemvBatch and
@@ -1419,6 +1458,11 @@ __global__ __launch_bounds__(NT) void gemv_lds_kernel(
     const int lane = tid & 63;
     const int col = lane % CW;
     const int slot = lane / CW;
+    // x first (the barrier waits for it), in passes of XB chunks per thread
+    uint4 xv[XB];
+#pragma unroll
+    for (int i = 0; i < XB; ++i) xv[i] = x[std::min(tid + i * NT, nchunks - 1)];
+    __builtin_amdgcn_sched_barrier(0);
     const uint32_t blk = xcd_block<xcd_run(JB)>();
     const int64_t row =
         (static_cast<int64_t>(blk) * (NT >> 6) + (tid >> 6)) * SLOTS + slot;
@@ -1427,11 +1471,6 @@ __global__ __launch_bounds__(NT) void gemv_lds_kernel(
     const uint32_t wrow_bytes = static_cast<uint32_t>(nchunks) * 16u;
     const int nbatch = ((nchunks + CW - 1) / CW + JB - 1) / JB;
 
-    // x first (the barrier waits for it), in passes of XB chunks per thread
-    uint4 xv[XB];
-#pragma unroll
-    for (int i = 0; i < XB; ++i) xv[i] = x[std::min(tid + i * NT, nchunks - 1)];
-    __builtin_amdgcn_sched_barrier(0);
     uint4 wa[JB], wn[JB];
     auto load = [&](uint4 (&dst)[JB], int b) {
 #pragma unroll
@@ -1440,6 +1479,7 @@ __global__ __launch_bounds__(NT) void gemv_lds_kernel(
             const uint32_t cl = static_cast<uint32_t>(c < nchunks ? c : nchunks - 1);
             dst[jj] = *reinterpret_cast<const uint4*>(wb + (rowc * wrow_bytes + cl * 16u));
         }
+        __builtin_amdgcn_sched_barrier(0);
     };
     load(wa, 0);
     __builtin_amdgcn_sched_barrier(0);
@@ -1463,13 +1503,19 @@ __global__ __launch_bounds__(NT) void gemv_lds_kernel(
             dot_chunk(S{}, src[jj], xs[c < nchunks ? c : nchunks], accs);
         }
     };
-    for (int b = 0; b < nbatch; b += 2) {
-        if (b + 1 < nbatch) load(wn, b + 1);
+    int b = 0;
+    for (; b + 2 < nbatch; b += 2) {
+        load(wn, b + 1);
         comp(wa, b);
-        if (b + 1 < nbatch) {
-            if (b + 2 < nbatch) load(wa, b + 2);
-            comp(wn, b + 1);
-        }
+        load(wa, b + 2);
+        comp(wn, b + 1);
+    }
+    if (b + 1 < nbatch) {
+        load(wn, b + 1);
+        comp(wa, b);
+        comp(wn, b + 1);
+    } else {
+        comp(wa, b);
     }
     float acc = (accs[0] + accs[1]) + (accs[2] + accs[3]);
     acc = segment_sum<CW>(acc);
