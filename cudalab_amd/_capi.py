@@ -73,6 +73,12 @@ class CqProblem(ctypes.Structure):
     ]
 
 
+class CqRepeat(ctypes.Structure):
+    """cq_repeat_t: a second copy of one problem's output, runs repeated."""
+    _fields_ = [("problem", ctypes.c_int64), ("y", ctypes.c_void_p),
+                ("head", ctypes.c_int64), ("times", ctypes.c_int64)]
+
+
 class CqPrepared(ctypes.Structure):
     """cq_prepared_t: a launch resolved by cq_prepare (opaque)."""
     _fields_ = [("opaque", ctypes.c_uint64 * 12)]
@@ -92,6 +98,10 @@ SIGNATURES = {
                                            _i64, _i64, _vp]),
     "cq_qgemv_grouped": (ctypes.c_int, [_cstr, ctypes.POINTER(CqProblem),
                                         _i64, _i64, _vp]),
+    "cq_int4gemv_grouped_repeat": (ctypes.c_int, [
+        _cstr, ctypes.POINTER(CqProblem), _i64, _i64, ctypes.POINTER(CqRepeat), _vp]),
+    "cq_qgemv_grouped_repeat": (ctypes.c_int, [
+        _cstr, ctypes.POINTER(CqProblem), _i64, _i64, ctypes.POINTER(CqRepeat), _vp]),
     "cq_int4_quantize": (ctypes.c_int, [_vp, _vp, _vp, _i64, _i64,
                                         ctypes.c_int, _vp]),
     "cq_q8_quantize": (ctypes.c_int, [_vp, _vp, _vp, _i64, _i64,

@@ -324,7 +324,7 @@ int check_quantize(int op, const void* w, const void* q, const void* scale,
 }
 
 int run_grouped(int op, const char* variant, const cq_gemv_problem_t* probs,
-                int64_t count, int64_t k, void* stream) {
+                int64_t count, int64_t k, const cq_repeat_t* repeat, void* stream) {
     g_last_error.clear();
     if (probs == nullptr) return fail(CQ_ERR_INVALID_ARG, "problems is NULL");
     if (count < 1 || count > INT_MAX)
@@ -375,6 +375,21 @@ int run_grouped(int op, const char* variant, const cq_gemv_problem_t* probs,
                 if (*it != j && overlaps(ys(*it), *sp)) return conflict(*it, what, j);
         }
     }
+    if (repeat != nullptr) {
+        const cq_repeat_t& r = *repeat;
+        if (r.problem < 0 || r.problem >= count || r.y == nullptr || r.head < 1 ||
+            r.times < 1 || probs[r.problem].n % r.head != 0 ||
+            r.times > INT_MAX / probs[r.problem].n)
+            return fail(CQ_ERR_INVALID_ARG, "repeat: problem, y, head (a divisor of the "
+                                            "problem's n) or times out of range");
+        Span c;
+        c.lo = reinterpret_cast<uintptr_t>(r.y);
+        c.hi = c.lo + static_cast<unsigned __int128>(probs[r.problem].n * r.times) * 2;
+        for (const Operands& o : ops)
+            if (overlaps(c, o.w) || overlaps(c, o.scale) || overlaps(c, o.x) || overlaps(c, o.y))
+                return fail(CQ_ERR_INVALID_ARG, "repeat: y overlaps an operand of the group");
+    }
+    bool repeated = false;
     hipStream_t s = static_cast<hipStream_t>(stream);
     auto one = [&](const cq_gemv_problem_t& q) {
         const cq::Plan p = make_plan(op, *v, q.n, k, q.w, q.x);
@@ -393,12 +408,26 @@ int run_grouped(int op, const char* variant, const cq_gemv_problem_t* probs,
             p = op == CQ_OP_INT4GEMV ? cq::plan_int4_group(v->rows, gp, c, k)
                                      : cq::plan_q8_group(v->rows, gp, c, k);
         if (v->kind == cq::kLds && p.kind == cq::kLds) {
-            e = op == CQ_OP_INT4GEMV ? cq::launch_int4_group(p, gp, c, k, s)
-                                     : cq::launch_q8_group(p, gp, c, k, s);
+            cq::Repeat rep{};
+            const bool here = repeat != nullptr && repeat->problem >= off &&
+                              repeat->problem < off + c;
+            if (here)
+                rep = {repeat->y, static_cast<int>(repeat->problem - off),
+                       static_cast<int>(repeat->head), static_cast<int>(repeat->times)};
+            const cq::Repeat* rp = here ? &rep : nullptr;
+            e = op == CQ_OP_INT4GEMV ? cq::launch_int4_group(p, gp, c, k, rp, &repeated, s)
+                                     : cq::launch_q8_group(p, gp, c, k, rp, &repeated, s);
         } else {
             for (int i = 0; i < c && e == hipSuccess; ++i) e = one(probs[off + i]);
         }
         if (e != hipSuccess) return hip_fail(e, "grouped launch");
+    }
+    if (repeat != nullptr && !repeated) {
+        const cq_gemv_problem_t& q = probs[repeat->problem];
+        const cq::Repeat rep{repeat->y, 0, static_cast<int>(repeat->head),
+                             static_cast<int>(repeat->times)};
+        const hipError_t e = cq::launch_repeat(q.y, q.n, rep, s);
+        if (e != hipSuccess) return hip_fail(e, "repeat launch");
     }
     return CQ_OK;
 }
@@ -536,12 +565,24 @@ int cq_gemv(const char* variant, int dtype, const void* w, const void* x,
 
 int cq_int4gemv_grouped(const char* variant, const cq_gemv_problem_t* problems,
                         int64_t n_problems, int64_t k, void* stream) {
-    return run_grouped(CQ_OP_INT4GEMV, variant, problems, n_problems, k, stream);
+    return run_grouped(CQ_OP_INT4GEMV, variant, problems, n_problems, k, nullptr, stream);
 }
 
 int cq_qgemv_grouped(const char* variant, const cq_gemv_problem_t* problems,
                      int64_t n_problems, int64_t k, void* stream) {
-    return run_grouped(CQ_OP_QGEMV, variant, problems, n_problems, k, stream);
+    return run_grouped(CQ_OP_QGEMV, variant, problems, n_problems, k, nullptr, stream);
+}
+
+int cq_int4gemv_grouped_repeat(const char* variant, const cq_gemv_problem_t* problems,
+                               int64_t n_problems, int64_t k, const cq_repeat_t* repeat,
+                               void* stream) {
+    return run_grouped(CQ_OP_INT4GEMV, variant, problems, n_problems, k, repeat, stream);
+}
+
+int cq_qgemv_grouped_repeat(const char* variant, const cq_gemv_problem_t* problems,
+                            int64_t n_problems, int64_t k, const cq_repeat_t* repeat,
+                            void* stream) {
+    return run_grouped(CQ_OP_QGEMV, variant, problems, n_problems, k, repeat, stream);
 }
 
 int cq_int4_quantize(const void* w, void* w_packed, void* scale, int64_t n,

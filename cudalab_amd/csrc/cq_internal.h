@@ -104,10 +104,21 @@ struct GroupProblem {
 // problems one by one" (each then gets its own plan).  `rows` as above.
 Plan plan_int4_group(int rows, const GroupProblem* probs, int count, int64_t k);
 Plan plan_q8_group(int rows, const GroupProblem* probs, int count, int64_t k);
+// A second copy of one problem's output: every run of `head` rows `times`
+// times in a row (problem counts from the launch's first).
+struct Repeat {
+    void* y;
+    int problem, head, times;
+};
+// `rep` (null for none) is written by the launch where its kernel can, and
+// *repeated says so; else the caller runs launch_repeat on the output.
 hipError_t launch_int4_group(const Plan& plan, const GroupProblem* probs,
-                             int count, int64_t k, hipStream_t stream);
+                             int count, int64_t k, const Repeat* rep, bool* repeated,
+                             hipStream_t stream);
 hipError_t launch_q8_group(const Plan& plan, const GroupProblem* probs,
-                           int count, int64_t k, hipStream_t stream);
+                           int count, int64_t k, const Repeat* rep, bool* repeated,
+                           hipStream_t stream);
+hipError_t launch_repeat(const void* src, int64_t n, const Repeat& rep, hipStream_t stream);
 
 // FP16/FP32 GEMV (the reference's kernels/gemv): element type of W, x, y.
 enum Dtype : int { kF16 = 0, kF32 = 1 };

@@ -689,7 +689,7 @@ struct RowSlot {
 
 // Operands of a launch of one problem; the grouped kernels have their own.
 // `slot()` is evaluated behind the x loads, `scale` behind the first weight
-// load, `y` at the end: none holds back a load that does not need it.
+// load, `store` at the end: none holds back a load that does not need it.
 template <typename S, uint32_t RUN>
 struct OneProblem {
     const uint4* w_;
@@ -699,7 +699,9 @@ struct OneProblem {
     __device__ __forceinline__ RowSlot slot() const { return {0, xcd_block<RUN>(), n_}; }
     __device__ __forceinline__ const uint4* w(const RowSlot&) const { return w_; }
     __device__ __forceinline__ const S* scale(const RowSlot&) const { return scale_; }
-    __device__ __forceinline__ uint16_t* y(const RowSlot&) const { return y_; }
+    __device__ __forceinline__ void store(const RowSlot&, int64_t row, uint16_t v) const {
+        y_[row] = v;
+    }
 };
 
 // One workgroup's rows of one INT4 problem.  `xs` is the workgroup's LDS:
@@ -851,7 +853,7 @@ __device__ __forceinline__ void int4_lds_rows(
         }
         acc = segment_sum<CW>(acc);
         const int64_t row = row0 + SLOTS * r;
-        if (col == CW - 1 && row < n) ops.y(g)[row] = f2h(acc);
+        if (col == CW - 1 && row < n) ops.store(g, row, f2h(acc));
     }
     if constexpr (STAMP) {
         __builtin_amdgcn_sched_barrier(0);
@@ -962,7 +964,7 @@ __device__ __forceinline__ void q8_lds_rows(
         }
         acc = segment_sum<CW>(acc);
         const int64_t row = row0 + SLOTS * r;
-        if (col == CW - 1 && row < n) ops.y(g)[row] = f2h(sc[r] * acc);
+        if (col == CW - 1 && row < n) ops.store(g, row, f2h(sc[r] * acc));
     }
 }
 
@@ -1298,13 +1300,26 @@ __device__ __forceinline__ RowSlot group_slot(const int (&n)[COUNT]) {
     return s;
 }
 
-// Two or three problems with one x.
-template <typename S, int ROWS, uint32_t RUN>
+// A second copy of problem p's output with every run of 2^shift rows (a head)
+// written `times` times in a row.  It is written with the rows themselves: a
+// decode step that repeats v for its query heads paid a copy launch of its own
+// for it (two 70B layers as a graph 165.9 us with the copy, 159.4 without).
+struct RepeatRows {
+    uint16_t* y;
+    int p, shift, times;
+};
+
+// Up to three problems with one x.  Rep is RepeatRows, or NoRepeat in the
+// kernels without a second copy (its test and arguments cost the other groups
+// 0.02-0.05 us a launch).
+struct NoRepeat {};
+template <typename S, int ROWS, uint32_t RUN, class Rep>
 struct Group3 {
     const uint4* w_[3];
     const S* scale_[3];
     uint16_t* y_[3];
     int n_[3];
+    Rep rep_;
     __device__ __forceinline__ RowSlot slot() const { return group_slot<ROWS, RUN>(n_); }
     __device__ __forceinline__ const uint4* w(const RowSlot& s) const {
         return pick3(s.p, w_[0], w_[1], w_[2]);
@@ -1312,8 +1327,15 @@ struct Group3 {
     __device__ __forceinline__ const S* scale(const RowSlot& s) const {
         return pick3(s.p, scale_[0], scale_[1], scale_[2]);
     }
-    __device__ __forceinline__ uint16_t* y(const RowSlot& s) const {
-        return pick3(s.p, y_[0], y_[1], y_[2]);
+    __device__ __forceinline__ void store(const RowSlot& s, int64_t row, uint16_t v) const {
+        pick3(s.p, y_[0], y_[1], y_[2])[row] = v;
+        if constexpr (std::is_same_v<Rep, RepeatRows>) {
+            if (s.p != rep_.p) return;
+            const int64_t head = row >> rep_.shift;
+            uint16_t* y = rep_.y + ((head * rep_.times) << rep_.shift) +
+                          (row - (head << rep_.shift));
+            for (int t = 0; t < rep_.times; ++t) y[static_cast<int64_t>(t) << rep_.shift] = v;
+        }
     }
 };
 
@@ -1327,7 +1349,9 @@ struct OneSlot {
     __device__ __forceinline__ RowSlot slot() const { return s_; }
     __device__ __forceinline__ const uint4* w(const RowSlot&) const { return w_; }
     __device__ __forceinline__ const S* scale(const RowSlot&) const { return scale_; }
-    __device__ __forceinline__ uint16_t* y(const RowSlot&) const { return y_; }
+    __device__ __forceinline__ void store(const RowSlot&, int64_t row, uint16_t v) const {
+        y_[row] = v;
+    }
 };
 
 struct GroupRecord {
@@ -1340,16 +1364,16 @@ struct Group8Records {
     GroupRecord r[kMaxGroup];
 };
 
-template <int CW, int J, int R, int NT>
+template <int CW, int J, int R, int NT, class Rep>
 __global__ __launch_bounds__(NT) void int4gemv_lds_group3_kernel(
         const uint4* x, const uint4* w0, const uint4* w1, const uint4* w2, int n0,
         int n1, int n2, int nchunks, const uint16_t* s0, const uint16_t* s1, const uint16_t* s2,
-        uint16_t* y0, uint16_t* y1, uint16_t* y2) {
+        uint16_t* y0, uint16_t* y1, uint16_t* y2, Rep rep) {
     extern __shared__ uint4 xs[];
     constexpr int kRows = 64 / CW * R * (NT / 64);
     int4_lds_rows<CW, J, R, NT>(x, nchunks, xs,
-        Group3<uint16_t, kRows, xcd_run(J * R)>{{w0, w1, w2}, {s0, s1, s2}, {y0, y1, y2},
-                                          {n0, n1, n2}});
+        Group3<uint16_t, kRows, xcd_run(J * R), Rep>{{w0, w1, w2}, {s0, s1, s2}, {y0, y1, y2},
+                                               {n0, n1, n2}, rep});
 }
 
 template <int CW, int J, int R, int NT>
@@ -1365,16 +1389,16 @@ __global__ __launch_bounds__(NT) void int4gemv_lds_group8_kernel(
                     static_cast<uint16_t*>(r.y), s});
 }
 
-template <int CW, int J, int R, int NT>
+template <int CW, int J, int R, int NT, class Rep>
 __global__ __launch_bounds__(NT) void qgemv_lds_group3_kernel(
         const uint4* x, const uint4* w0, const uint4* w1, const uint4* w2, int n0,
         int n1, int n2, int nchunks, const float* s0, const float* s1, const float* s2,
-        uint16_t* y0, uint16_t* y1, uint16_t* y2) {
+        uint16_t* y0, uint16_t* y1, uint16_t* y2, Rep rep) {
     extern __shared__ uint4 xs[];
     constexpr int kRows = 64 / CW * R * (NT / 64);
     q8_lds_rows<CW, J, R, NT>(x, nchunks, xs,
-        Group3<float, kRows, xcd_run(J * R)>{{w0, w1, w2}, {s0, s1, s2}, {y0, y1, y2},
-                                          {n0, n1, n2}});
+        Group3<float, kRows, xcd_run(J * R), Rep>{{w0, w1, w2}, {s0, s1, s2}, {y0, y1, y2},
+                                               {n0, n1, n2}, rep});
 }
 
 template <int CW, int J, int R, int NT>
@@ -1597,6 +1621,18 @@ __global__ __launch_bounds__(NT) void gemv_tiled_kernel(
     if (col == 63 && row < n) fp_store(y + row, acc);
 }
 
+// The copy RepeatRows describes, for outputs the grouped kernels did not
+// write it with.
+__global__ __launch_bounds__(kBlock) void repeat_rows_kernel(
+        const uint16_t* __restrict__ src, uint16_t* __restrict__ dst, int n, int head,
+        int times) {
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+    if (i >= n) return;
+    const int64_t h = i / head;
+    const uint16_t v = src[i];
+    for (int t = 0; t < times; ++t) dst[(h * times + t) * head + (i - h * head)] = v;
+}
+
 // ------------------------------------------------- read-only ceiling
 //
 // A plain streaming read of `bytes`, one 16-byte load per thread.  Of the
@@ -1712,19 +1748,19 @@ struct Int4LdsStamp {
     }
 };
 
-template <typename S>
+template <typename S, class Rep>
 using Group3Fn = void (*)(const uint4*, const uint4*, const uint4*, const uint4*, int,
                           int, int, int, const S*, const S*, const S*, uint16_t*,
-                          uint16_t*, uint16_t*);
+                          uint16_t*, uint16_t*, Rep);
 using Group8Fn = void (*)(int, int, int, int, int, int, int, int, int, Group8Records);
 
-template <int NT>
+template <int NT, class Rep>
 struct Int4LdsGroup3 {
-    using Fn = Group3Fn<uint16_t>;
+    using Fn = Group3Fn<uint16_t, Rep>;
     static constexpr int kMaxJ = kInt4MaxJ;
     template <int CW, int J, int R>
     static constexpr Fn get() {
-        if constexpr (R <= int4_rmax(J)) return &int4gemv_lds_group3_kernel<CW, J, R, NT>;
+        if constexpr (R <= int4_rmax(J)) return &int4gemv_lds_group3_kernel<CW, J, R, NT, Rep>;
         else return nullptr;
     }
 };
@@ -1738,13 +1774,13 @@ struct Int4LdsGroup8 {
         else return nullptr;
     }
 };
-template <int NT>
+template <int NT, class Rep>
 struct Q8LdsGroup3 {
-    using Fn = Group3Fn<float>;
+    using Fn = Group3Fn<float, Rep>;
     static constexpr int kMaxJ = kQ8MaxJ;
     template <int CW, int J, int R>
     static constexpr Fn get() {
-        if constexpr (R <= q8_rmax(J)) return &qgemv_lds_group3_kernel<CW, J, R, NT>;
+        if constexpr (R <= q8_rmax(J)) return &qgemv_lds_group3_kernel<CW, J, R, NT, Rep>;
         else return nullptr;
     }
 };
@@ -2148,13 +2184,13 @@ Plan group_plan(PlanFn plan_one, OkFn lds_ok, int rows,
     return p;
 }
 
-// One grouped launch of plan `p`: the kernel for two or three problems that
+// One grouped launch of plan `p`: the kernel for up to three problems that
 // share x, or the general one.  An absent problem has no rows.
-template <typename S>
-hipError_t launch_group(Group3Fn<S> fn3, Group8Fn fn8, const Plan& p,
-                        const GroupProblem* probs, int count, uint32_t shmem,
-                        int nchunks, hipStream_t stream) {
-    if (fn3 == nullptr || fn8 == nullptr) return hipErrorInvalidConfiguration;
+template <typename S, template <int, class> class F3, template <int> class F8>
+hipError_t launch_group(const Plan& p, const GroupProblem* probs, int count,
+                        uint32_t shmem, int nchunks, const Repeat* rep, bool* repeated,
+                        hipStream_t stream) {
+    const bool wide = p.block == 512;
     const int64_t rows = static_cast<int64_t>(64 / p.cw) * p.r * (p.block / 64);
     int64_t grid = 0;
     int n[kMaxGroup] = {};
@@ -2174,14 +2210,29 @@ hipError_t launch_group(Group3Fn<S> fn3, Group8Fn fn8, const Plan& p,
             sc[i] = static_cast<const S*>(probs[i].scale);
             y[i] = static_cast<uint16_t*>(probs[i].y);
         }
-        return launch(fn3, grid, p.block, shmem, stream, nullptr, nullptr,
-                      static_cast<const uint4*>(probs[0].x), w[0], w[1], w[2], n[0], n[1],
-                      n[2], nchunks, sc[0], sc[1], sc[2], y[0], y[1], y[2]);
+        auto go = [&](auto fn, auto r) {
+            if (fn == nullptr) return hipErrorInvalidConfiguration;
+            return launch(fn, grid, p.block, shmem, stream, nullptr, nullptr,
+                          static_cast<const uint4*>(probs[0].x), w[0], w[1], w[2], n[0],
+                          n[1], n[2], nchunks, sc[0], sc[1], sc[2], y[0], y[1], y[2], r);
+        };
+        if (rep != nullptr && (rep->head & (rep->head - 1)) == 0) {
+            RepeatRows r{static_cast<uint16_t*>(rep->y), rep->problem, 0, rep->times};
+            while ((1 << r.shift) < rep->head) ++r.shift;
+            *repeated = true;
+            return go(wide ? instance<F3<512, RepeatRows>>(p.cw, p.j, p.r)
+                           : instance<F3<kBlock, RepeatRows>>(p.cw, p.j, p.r), r);
+        }
+        return go(wide ? instance<F3<512, NoRepeat>>(p.cw, p.j, p.r)
+                       : instance<F3<kBlock, NoRepeat>>(p.cw, p.j, p.r), NoRepeat{});
     }
+    const Group8Fn fn = wide ? instance<F8<512>>(p.cw, p.j, p.r)
+                             : instance<F8<kBlock>>(p.cw, p.j, p.r);
+    if (fn == nullptr) return hipErrorInvalidConfiguration;
     Group8Records g = {};
     for (int i = 0; i < count; ++i)
         g.r[i] = {probs[i].w, probs[i].scale, probs[i].x, probs[i].y};
-    return launch(fn8, grid, p.block, shmem, stream, nullptr, nullptr, n[0], n[1], n[2],
+    return launch(fn, grid, p.block, shmem, stream, nullptr, nullptr, n[0], n[1], n[2],
                   n[3], n[4], n[5], n[6], n[7], nchunks, g);
 }
 
@@ -2208,29 +2259,23 @@ Plan plan_q8_group(int rows, const GroupProblem* probs, int count, int64_t k) {
 }
 
 hipError_t launch_int4_group(const Plan& p, const GroupProblem* probs,
-                             int count, int64_t k, hipStream_t stream) {
+                             int count, int64_t k, const Repeat* rep,
+                             bool* repeated, hipStream_t stream) {
     if (p.kind != kLds || count < 1 || count > kMaxGroup || !lds_chunks_ok(p, k / 32))
         return hipErrorInvalidConfiguration;
-    const bool wide = p.block == 512;
-    return launch_group(wide ? instance<Int4LdsGroup3<512>>(p.cw, p.j, p.r)
-                             : instance<Int4LdsGroup3<kBlock>>(p.cw, p.j, p.r),
-                        wide ? instance<Int4LdsGroup8<512>>(p.cw, p.j, p.r)
-                             : instance<Int4LdsGroup8<kBlock>>(p.cw, p.j, p.r),
-                        p, probs, count, int4_lds_bytes(p.cw, p.j),
-                        static_cast<int>(k / 32), stream);
+    return launch_group<uint16_t, Int4LdsGroup3, Int4LdsGroup8>(
+        p, probs, count, int4_lds_bytes(p.cw, p.j), static_cast<int>(k / 32), rep, repeated,
+        stream);
 }
 
 hipError_t launch_q8_group(const Plan& p, const GroupProblem* probs,
-                             int count, int64_t k, hipStream_t stream) {
+                             int count, int64_t k, const Repeat* rep,
+                             bool* repeated, hipStream_t stream) {
     if (p.kind != kLds || count < 1 || count > kMaxGroup || !lds_chunks_ok(p, k / 16))
         return hipErrorInvalidConfiguration;
-    const bool wide = p.block == 512;
-    return launch_group(wide ? instance<Q8LdsGroup3<512>>(p.cw, p.j, p.r)
-                             : instance<Q8LdsGroup3<kBlock>>(p.cw, p.j, p.r),
-                        wide ? instance<Q8LdsGroup8<512>>(p.cw, p.j, p.r)
-                             : instance<Q8LdsGroup8<kBlock>>(p.cw, p.j, p.r),
-                        p, probs, count, q8_lds_bytes(p.cw, p.j),
-                        static_cast<int>(k / 16), stream);
+    return launch_group<float, Q8LdsGroup3, Q8LdsGroup8>(
+        p, probs, count, q8_lds_bytes(p.cw, p.j), static_cast<int>(k / 16), rep, repeated,
+        stream);
 }
 
 // ---- FP16/FP32 GEMV
@@ -2341,6 +2386,12 @@ hipError_t launch_gemv(const Plan& p, int dtype, const void* w, const void* x,
     Launch L;
     const hipError_t e = prepare_gemv(p, dtype, w, x, y, n, k, &L);
     return e != hipSuccess ? e : enqueue(L, stream, ev0, ev1);
+}
+
+hipError_t launch_repeat(const void* src, int64_t n, const Repeat& rep, hipStream_t stream) {
+    return launch(repeat_rows_kernel, (n + kBlock - 1) / kBlock, kBlock, 0, stream, nullptr,
+                  nullptr, static_cast<const uint16_t*>(src), static_cast<uint16_t*>(rep.y),
+                  static_cast<int>(n), rep.head, rep.times);
 }
 
 hipError_t launch_stream_read(const void* buf, int64_t bytes, void* sink,

@@ -56,6 +56,8 @@ using PrepareFn = int (*)(int, const char*, const void*, const void*, const void
 using LaunchFn = int (*)(const cq_prepared_t*, void*);
 using ErrorFn = const char* (*)();
 using GroupedFn = int (*)(const char*, const cq_gemv_problem_t*, int64_t, int64_t, void*);
+using RepeatFn = int (*)(const char*, const cq_gemv_problem_t*, int64_t, int64_t,
+                         const cq_repeat_t*, void*);
 
 enum Kind { kInt4 = 0, kQ8 = 1, kGemv = 2 };
 
@@ -112,12 +114,13 @@ class Launcher {
 public:
     Launcher(int kind, const std::vector<std::string>& names, uintptr_t prepare,
              uintptr_t launch, uintptr_t last_error, int64_t capacity,
-             uintptr_t grouped)
+             uintptr_t grouped, uintptr_t grouped_repeat)
         : kind_(kind),
           prepare_(reinterpret_cast<PrepareFn>(prepare)),
           launch_(reinterpret_cast<LaunchFn>(launch)),
           last_error_(reinterpret_cast<ErrorFn>(last_error)),
           grouped_(reinterpret_cast<GroupedFn>(grouped)),
+          grouped_repeat_(reinterpret_cast<RepeatFn>(grouped_repeat)),
           capacity_(capacity < 1 ? 1 : static_cast<size_t>(capacity)),
           names_(names) {
         if (kind < kInt4 || kind > kGemv) throw std::invalid_argument("unknown operator kind");
@@ -196,8 +199,31 @@ public:
     // checks (overlaps included); a refusal there is "not taken" too, so
     // the checked path raises it with the reference-style message.
     bool grouped(py::handle variant, py::handle problems) {
+        if (grouped_ == nullptr) return false;
+        return run_grouped(variant, problems, nullptr);
+    }
+    // The same with a second copy of problem `index`'s output into `out`,
+    // each run of `head` outputs repeated (cq_*_grouped_repeat).
+    bool grouped_repeat(py::handle variant, py::handle problems, int64_t index,
+                        py::handle out, int64_t head) {
+        if (grouped_repeat_ == nullptr || !THPVariable_Check(out.ptr())) return false;
+        const RepeatTo to{index, &THPVariable_Unpack(out.ptr()), head};
+        return run_grouped(variant, problems, &to);
+    }
+
+    bool knows(py::handle variant) const { return variant_id(variant) >= 0; }
+    size_t cached() const { return cache_.size(); }
+    void clear() { cache_.clear(); }
+
+private:
+    struct RepeatTo {
+        int64_t index;
+        const at::Tensor* out;
+        int64_t head;
+    };
+    bool run_grouped(py::handle variant, py::handle problems, const RepeatTo* to) {
         const int32_t vid = variant_id(variant);
-        if (vid < 0 || kind_ == kGemv || grouped_ == nullptr) return false;
+        if (vid < 0 || kind_ == kGemv) return false;
         PyObject* seq = problems.ptr();
         if (!PyList_Check(seq) && !PyTuple_Check(seq)) return false;
         const Py_ssize_t count = PySequence_Fast_GET_SIZE(seq);
@@ -229,8 +255,21 @@ public:
                                              Y.data_ptr(), W.size(0)};
         }
         const hipStream_t stream = c10::hip::getCurrentHIPStream(dev0.index()).stream();
-        const int st = grouped_(names_[static_cast<size_t>(vid)].c_str(), probs.data(),
-                                static_cast<int64_t>(count), k0, stream);
+        const char* name = names_[static_cast<size_t>(vid)].c_str();
+        int st;
+        if (to != nullptr) {
+            if (to->index < 0 || to->index >= count) return false;
+            const int64_t n = probs[static_cast<size_t>(to->index)].n;
+            const at::Tensor& o = *to->out;
+            if (!plain(o, at::kHalf) || o.dim() != 1 || o.device() != dev0 || to->head < 1 ||
+                o.size(0) < n || o.size(0) % n != 0 || n % to->head != 0)
+                return false;
+            const cq_repeat_t rep{to->index, o.data_ptr(), to->head, o.size(0) / n};
+            st = grouped_repeat_(name, probs.data(), static_cast<int64_t>(count), k0, &rep,
+                                 stream);
+        } else {
+            st = grouped_(name, probs.data(), static_cast<int64_t>(count), k0, stream);
+        }
         if (st == CQ_OK) return true;
         if (st == CQ_ERR_HIP)
             throw std::runtime_error(std::string(kind_ == kInt4 ? "int4gemv" : "qgemv") +
@@ -239,11 +278,6 @@ public:
         return false;
     }
 
-    bool knows(py::handle variant) const { return variant_id(variant) >= 0; }
-    size_t cached() const { return cache_.size(); }
-    void clear() { cache_.clear(); }
-
-private:
     static bool all_tensors(std::initializer_list<py::handle> objs) {
         for (py::handle o : objs)
             if (!THPVariable_Check(o.ptr())) return false;
@@ -333,6 +367,7 @@ private:
     LaunchFn launch_;
     ErrorFn last_error_;
     GroupedFn grouped_;
+    RepeatFn grouped_repeat_;
     size_t capacity_;
     std::vector<std::string> names_;
     std::unordered_map<std::string_view, int32_t> ids_;
@@ -347,9 +382,10 @@ PYBIND11_MODULE(_cqfast, m) {
     m.attr("abi_stamp") = CQ_FAST_ABI;   // torch version, C++ ABI, g++ flags
     py::class_<Launcher>(m, "Launcher")
         .def(py::init<int, const std::vector<std::string>&, uintptr_t, uintptr_t,
-                      uintptr_t, int64_t, uintptr_t>(),
+                      uintptr_t, int64_t, uintptr_t, uintptr_t>(),
              py::arg("kind"), py::arg("names"), py::arg("prepare"), py::arg("launch"),
-             py::arg("last_error"), py::arg("capacity"), py::arg("grouped") = 0)
+             py::arg("last_error"), py::arg("capacity"), py::arg("grouped") = 0,
+             py::arg("grouped_repeat") = 0)
         .def("accepts", &Launcher::accepts)
         .def("gemv_accepts", &Launcher::gemv_accepts)
         .def("into", &Launcher::into)
@@ -357,6 +393,7 @@ PYBIND11_MODULE(_cqfast, m) {
         .def("gemv_into", &Launcher::gemv_into)
         .def("gemv_forward", &Launcher::gemv_forward)
         .def("grouped", &Launcher::grouped)
+        .def("grouped_repeat", &Launcher::grouped_repeat)
         .def("knows", &Launcher::knows)
         .def("cached", &Launcher::cached)
         .def("clear", &Launcher::clear);

@@ -12,7 +12,8 @@ grouped-query attention; Llama-70B: H = 8192, I = 28672, KV = 1024):
                                                  attention the identity on v;
                                                  with KV < H each kv head's v
                                                  is repeated for its H/KV
-                                                 query heads, one small copy)
+                                                 query heads, written by v's
+                                                 own launch)
   gate, up  H -> I   from o                     (independent: one group)
   down      I -> H   from up                    (feeds the next layer)
 Norms, attention over a longer context, the residual adds and the SwiGLU
@@ -133,25 +134,25 @@ class DecodeModel:
         self.ext.forward_into(self.variant, W, s, x, L.out[name])
 
     def _group(self, L: Layer, names, x: torch.Tensor):
-        self.ext.forward_grouped(self.variant, [(L.w[n][0], L.w[n][1], x, L.out[n])
-                                                for n in names])
-
-    def _attend(self, L: Layer) -> torch.Tensor:
-        """Attention over a single-token context: each query head gets its
-        kv head's v (a copy when k/v are narrower than the hidden size)."""
-        if self.kv == self.hidden:
-            return L.out["v"]
-        kvh, rep = self.kv // HEAD_DIM, self.hidden // self.kv
-        L.out["o_in"].view(kvh, rep, HEAD_DIM).copy_(
-            L.out["v"].view(kvh, 1, HEAD_DIM).expand(kvh, rep, HEAD_DIM))
-        return L.out["o_in"]
+        problems = [(L.w[n][0], L.w[n][1], x, L.out[n]) for n in names]
+        if "v" in names and self.kv != self.hidden:
+            # attention over a single-token context: each query head gets its
+            # kv head's v
+            self.ext.forward_grouped_repeat(self.variant, problems, names.index("v"),
+                                            L.out["o_in"], HEAD_DIM)
+        else:
+            self.ext.forward_grouped(self.variant, problems)
 
     def step_sequential(self) -> torch.Tensor:
         x = self.x0
         for L in self.layers:
-            for n in ("q", "k", "v"):
+            for n in ("q", "k"):
                 self._one(L, n, x)
-            self._one(L, "o", self._attend(L))
+            if self.kv == self.hidden:
+                self._one(L, "v", x)
+            else:
+                self._group(L, ("v",), x)
+            self._one(L, "o", L.out["o_in"])
             for n in ("gate", "up"):
                 self._one(L, n, L.out["o"])
             self._one(L, "down", L.out["up"])
@@ -162,7 +163,7 @@ class DecodeModel:
         x = self.x0
         for L in self.layers:
             self._group(L, ("q", "k", "v"), x)
-            self._one(L, "o", self._attend(L))
+            self._one(L, "o", L.out["o_in"])
             self._group(L, ("gate", "up"), L.out["o"])
             self._one(L, "down", L.out["up"])
             x = L.out["down"]

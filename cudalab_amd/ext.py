@@ -72,7 +72,7 @@ class _DeclineAll:
     def accepts(self, *args) -> bool:
         return False
 
-    gemv_accepts = knows = into = gemv_into = grouped = accepts
+    gemv_accepts = knows = into = gemv_into = grouped = grouped_repeat = accepts
 
     def forward(self, *args):
         return None
@@ -107,7 +107,8 @@ def _fast_launcher(op: str, names: list[str]):
         _FAST_KIND[op], names, _capi.entry_address("cq_prepare"),
         _capi.entry_address("cq_launch_prepared"),
         _capi.entry_address("cq_last_error"), FAST_CACHE_ENTRIES,
-        _capi.entry_address(grouped) if grouped else 0)
+        _capi.entry_address(grouped) if grouped else 0,
+        _capi.entry_address(f"{grouped}_repeat") if grouped else 0)
 
 
 def _fail(msg: str) -> None:
@@ -134,6 +135,9 @@ class _OpExt:
         self._grouped_fn = (self._lib.cq_int4gemv_grouped
                             if self.op == "int4gemv"
                             else self._lib.cq_qgemv_grouped)
+        self._repeat_fn = (self._lib.cq_int4gemv_grouped_repeat
+                           if self.op == "int4gemv"
+                           else self._lib.cq_qgemv_grouped_repeat)
         self._fast = _fast_launcher(self.op, self._all + sorted(self._aliases))
 
     # ---- registry (bindings.cpp variant lists) ----
@@ -251,6 +255,46 @@ class _OpExt:
         if self._fast.grouped(variant, problems):
             return
         self._lookup(variant)
+        arr, K, dev = self._grouped_args(problems)
+        st = _on_device(dev, lambda stream: self._grouped_fn(
+            variant.encode(), arr, len(arr), K, stream))
+        if st != _capi.CQ_OK:
+            _fail(f"{self.op} grouped launch failed (status {st}): "
+                  f"{_capi.last_error()}")
+
+    def forward_grouped_repeat(self, variant: str, problems, index: int,
+                               out: torch.Tensor, head: int) -> None:
+        """forward_grouped that also writes problem `index`'s output into
+        `out` with each run of `head` outputs repeated: `out` is fp16 (N *
+        times,), out.view(N / head, times, head)[:, t] equals the output's
+        view(N / head, head) for every t.  In the group's own launch for up
+        to three problems with one x on the LDS variants (the decode step's
+        q/k/v with grouped-query v), by a copy behind it otherwise."""
+        if self._fast.grouped_repeat(variant, problems, index, out, head):
+            return
+        self._lookup(variant)
+        problems = list(problems)
+        arr, K, dev = self._grouped_args(problems)
+        if not 0 <= index < len(arr):
+            _fail(f"repeat index {index} names no problem of {len(arr)}")
+        n = arr[index].n
+        if out.dtype != torch.float16 or out.dim() != 1 or not out.is_contiguous() \
+                or out.device != dev:
+            _fail("the repeated output must be a contiguous 1-D float16 tensor on "
+                  "the weights' device")
+        if head < 1 or n % head != 0 or out.size(0) < n or out.size(0) % n != 0:
+            _fail(f"the repeated output has {out.size(0)} elements for {n} rows in "
+                  f"runs of {head}")
+        rep = _capi.CqRepeat(index, out.data_ptr(), head, out.size(0) // n)
+        st = _on_device(dev, lambda stream: self._repeat_fn(
+            variant.encode(), arr, len(arr), K, ctypes.byref(rep), stream))
+        if st != _capi.CQ_OK:
+            _fail(f"{self.op} grouped launch failed (status {st}): "
+                  f"{_capi.last_error()}")
+
+    def _grouped_args(self, problems):
+        """(problem array, K, device) of a grouped call, every problem
+        checked as forward_into checks its arguments."""
         problems = list(problems)
         if not problems:
             _fail("problems 不能为空 (problems must be a non-empty list)")
@@ -274,11 +318,7 @@ class _OpExt:
             arr[i].x = x.data_ptr()
             arr[i].y = out.data_ptr()
             arr[i].n = W.size(0)
-        st = _on_device(dev, lambda stream: self._grouped_fn(
-            variant.encode(), arr, len(problems), K, stream))
-        if st != _capi.CQ_OK:
-            _fail(f"{self.op} grouped launch failed (status {st}): "
-                  f"{_capi.last_error()}")
+        return arr, K, dev
 
     def native_timing(self, variant: str, W: torch.Tensor,
                       scale: torch.Tensor, x: torch.Tensor,
@@ -577,6 +617,9 @@ class GemvExt(_OpExt):
         self._launch2(variant, W, x, out)
 
     def forward_grouped(self, variant, problems):  # type: ignore[override]
+        _fail("gemv 不提供分组调用 (grouped calls exist for int4gemv and qgemv)")
+
+    def forward_grouped_repeat(self, variant, problems, index, out, head):
         _fail("gemv 不提供分组调用 (grouped calls exist for int4gemv and qgemv)")
 
     def native_timing(self, variant: str, W: torch.Tensor,  # type: ignore[override]

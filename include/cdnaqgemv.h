@@ -155,6 +155,31 @@ int cq_int4gemv_grouped(const char* variant, const cq_gemv_problem_t* problems,
 int cq_qgemv_grouped(const char* variant, const cq_gemv_problem_t* problems,
                      int64_t n_problems, int64_t k, void* stream);
 
+/* A second copy of one problem's output (cq_*_grouped_repeat). */
+typedef struct cq_repeat {
+    int64_t problem;   /* which problem's output */
+    void* y;           /* fp16, n * times elements */
+    int64_t head;      /* rows of a run; divides that problem's n */
+    int64_t times;     /* how often each run is written, one after another */
+} cq_repeat_t;
+
+/*
+ * cq_int4gemv_grouped / cq_qgemv_grouped that also write one output a second
+ * time with its runs repeated: y[(i / head * times + t) * head + i % head] of
+ * `repeat` receives output i for every t < times (grouped-query attention
+ * over one token hands each kv head's v to `times` query heads).  The copy
+ * shares no byte with any operand of the group.  Written by the grouped
+ * launch itself for up to three problems with one x on the LDS variants and a
+ * power-of-two head; by a copy behind it otherwise.  No counterpart in the
+ * reference.
+ */
+int cq_int4gemv_grouped_repeat(const char* variant, const cq_gemv_problem_t* problems,
+                               int64_t n_problems, int64_t k, const cq_repeat_t* repeat,
+                               void* stream);
+int cq_qgemv_grouped_repeat(const char* variant, const cq_gemv_problem_t* problems,
+                            int64_t n_problems, int64_t k, const cq_repeat_t* repeat,
+                            void* stream);
+
 /*
  * On-device INT4 quantize + pack of fp16 w [n, k] (k % 128 == 0) into
  * w_packed uint8 [n, k/2] and scale fp16 [n, k/128]: per group of 128,
