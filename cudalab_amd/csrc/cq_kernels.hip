@@ -141,9 +141,8 @@ __device__ __forceinline__ uint32_t xcd_block() { return xcd_block<RUN>(blockIdx
 // caches), once for its R rows.  Batches of U chunks run through two register
 // sets: batch b + 1 is in flight while batch b is summed (its loads are
 // unconditional, see gemv_lds_kernel).  The k % E elements past the last whole
-// chunk go one per lane.  Four accumulators per lane keep
-// the FMA chains as short as one element per thread of a 256-thread workgroup
-// would; the shares of a row meet in LDS and are added in wave order.  Chunks
+// chunk go one per lane.  Four accumulators per lane keep the FMA chains as
+// short as one element per thread of a 256-thread workgroup would; the shares of a row meet in LDS and are added in wave order.  Chunks
 // past the row end are re-read in bounds and not summed (no zero operand
 // stands in for them, so an infinite scale or x meets no extra product).
 //
@@ -652,10 +651,11 @@ __global__ __launch_bounds__(kBlock) void qgemv_wave_kernel(
 //   lives in scalar registers.
 // Issue order, pinned with scheduling barriers: the workgroup's x pieces,
 // then per row, chunk by chunk, the weight chunk and the group scale (the
-// grouped kernels know the weights' address before the scales'; INT8: the chunks, then the row scale), so that the wait before chunk j
-// covers chunks 0..j only and each chunk is summed as it lands.  A
-// scheduling barrier after the workgroup barrier keeps weight arithmetic
-// (and its waits) from being hoisted above it.
+// grouped kernels know the weights' address before the scales'; INT8: the
+// chunks, then the row scale), so that the wait before chunk j covers chunks
+// 0..j only and each chunk is summed as it lands.  A scheduling barrier after
+// the workgroup barrier keeps weight arithmetic (and its waits) from being
+// hoisted above it.
 
 // The timeline stamps pin their clock reads by data dependence, not by
 // scheduling fences (the compiler places pure arithmetic before the machine
@@ -1018,9 +1018,9 @@ __global__ __launch_bounds__(NT) void qgemv_lds_kernel(
 // per wave (CW = 64), both read against one copy of x.  x is staged tile by
 // tile: TJ * 64 chunks of the row per tile (TJ = 2..8: TJ * 2048 INT4 or
 // TJ * 1024 INT8 elements), re-paired in LDS, with a barrier before the
-// tile is read and one before the next tile overwrites it.  Every thread of the workgroup
-// runs the same tiles (they depend on nchunks only; rows past n are
-// clamped, never skipped), so every barrier is reached by all.  In the last,
+// tile is read and one before the next tile overwrites it.  Every thread of
+// the workgroup runs the same tiles (they depend on nchunks only; rows past n
+// are clamped, never skipped), so every barrier is reached by all.  In the last,
 // partial tile only the first ceil(tc / 64) chunks of each lane are loaded
 // and summed (a wave-uniform bound).  Lane `col` takes chunks col + 64 j of
 // its rows in j order, as the untiled kernels do, so each row's sum
@@ -1257,17 +1257,17 @@ constexpr uint32_t tile_lds(int pieces, int tj) {
 // arguments that the hardware preloads into scalar registers (the first 14
 // words), and the prefix sums of the workgroup counts are computed from the
 // row counts: a workgroup that first has to read a table from the argument
-// memory stands still for each dependent read (the table form
-// before cost 0.7-1.2 us a launch: four dependent reads):
-// - Group3 (two or three problems with one x: q/k/v, gate/up): x, the weights
+// memory stands still for each dependent read (a table cost 0.7-1.2 us a
+// launch: four dependent reads):
+// - Group3 (up to three problems with one x: q/k/v, gate/up): x, the weights
 //   and the row counts are preloaded; scale and y are read behind the first
 //   weight loads.
 // - Group8 (any other group): the row counts are preloaded; one 32-byte read
 //   brings the problem's pointers.
-// INT4 us per call, before and now (problems with one x): 3 x 4096x4096
-// 7.6 -> 6.4 (one matrix of the same rows 6.3), 2 x 11008x4096 10.9 -> 9.7,
-// 1024 + 256 + 256 x 1024 3.17 -> 2.22; with an x each: 3 x 4096x4096 6.7,
-// 1024 + 256 + 256 x 1024 2.54.
+// INT4 us per call, with the table and now (problems with one x): 3 x
+// 4096x4096 7.6 -> 6.4 (one matrix of the same rows 6.3), 2 x 11008x4096
+// 10.9 -> 9.7, 1024 + 256 + 256 x 1024 3.17 -> 2.22; with an x each: 3 x
+// 4096x4096 6.7, 1024 + 256 + 256 x 1024 2.54.
 constexpr int log2_of(int v) { return v <= 1 ? 0 : 1 + log2_of(v / 2); }
 
 // Selects of values: written on the arguments themselves, they would select
