@@ -1467,25 +1467,40 @@ __device__ __forceinline__ void dot_chunk(float, const uint4& w,
 // 3000x65536 67.2 us against 66.6.)
 constexpr int kGemvBatch = 8;
 
+// A chunk of x on its way to LDS is held as a vector: a uint4 that is only
+// copied is forwarded from x to LDS as one memory copy, which moves the load
+// behind the weight loads, and the barrier then waits for all of them (FP16
+// 4096^2 7.2 us that way, 6.5 with x first; 1024x4096 3.43, 2.88; 1000x30000
+// 15.7, 13.0; FP32 1000x30000 on the K-tiled kernel 33.5, 23.9).
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ u32x4 load_chunk(const uint4* p) {
+    return *reinterpret_cast<const u32x4*>(p);
+}
+__device__ __forceinline__ void store_chunk(uint4* p, u32x4 v) {
+    *reinterpret_cast<u32x4*>(p) = v;
+}
+
 // JB: chunks per lane per register batch, the smaller of kGemvBatch and
 // the lane's chunk count rounded up to a power of two (a batch longer than
-// the row would load and multiply padding).
-template <typename S, int CW, int NT, int JB>
+// the row would load and multiply padding).  ONE: the row is one batch; the
+// kernel is then a third of the size, and all of x is staged in one pass.
+template <typename S, int CW, int NT, int JB, bool ONE>
 __global__ __launch_bounds__(NT) void gemv_lds_kernel(
         const uint4* __restrict__ w,   // [n][nchunks] 16-byte chunks
         const uint4* __restrict__ x,   // [nchunks] 16-byte chunks
         S* __restrict__ y, int n, int nchunks) {
     extern __shared__ uint4 xs[];
     constexpr int SLOTS = 64 / CW;
-    constexpr int XB = 4;              // x chunks per thread per staging pass
+    // x chunks per thread per staging pass (all of x where the row is one batch)
+    constexpr int XB = ONE ? (CW * JB + NT - 1) / NT : 4;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int col = lane % CW;
     const int slot = lane / CW;
     // x first (the barrier waits for it), in passes of XB chunks per thread
-    uint4 xv[XB];
+    u32x4 xv[XB];
 #pragma unroll
-    for (int i = 0; i < XB; ++i) xv[i] = x[std::min(tid + i * NT, nchunks - 1)];
+    for (int i = 0; i < XB; ++i) xv[i] = load_chunk(x + std::min(tid + i * NT, nchunks - 1));
     __builtin_amdgcn_sched_barrier(0);
     const uint32_t blk = xcd_block<xcd_run(JB)>();
     const int64_t row =
@@ -1495,7 +1510,7 @@ __global__ __launch_bounds__(NT) void gemv_lds_kernel(
     const uint32_t wrow_bytes = static_cast<uint32_t>(nchunks) * 16u;
     const int nbatch = ((nchunks + CW - 1) / CW + JB - 1) / JB;
 
-    uint4 wa[JB], wn[JB];
+    uint4 wa[JB];
     auto load = [&](uint4 (&dst)[JB], int b) {
 #pragma unroll
         for (int jj = 0; jj < JB; ++jj) {
@@ -1508,13 +1523,15 @@ __global__ __launch_bounds__(NT) void gemv_lds_kernel(
     load(wa, 0);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int i = 0; i < XB; ++i) xs[std::min(tid + i * NT, nchunks - 1)] = xv[i];
-    for (int base = XB * NT; base < nchunks; base += XB * NT) {   // K beyond one pass
+    for (int i = 0; i < XB; ++i) store_chunk(xs + std::min(tid + i * NT, nchunks - 1), xv[i]);
+#pragma unroll 1
+    for (int base = XB * NT; !ONE && base < nchunks; base += XB * NT) {   // K beyond one pass
 #pragma unroll
-        for (int i = 0; i < XB; ++i) {
-            const int c = std::min(base + tid + i * NT, nchunks - 1);
-            xs[c] = x[c];
-        }
+        for (int i = 0; i < XB; ++i)
+            xv[i] = load_chunk(x + std::min(base + tid + i * NT, nchunks - 1));
+#pragma unroll
+        for (int i = 0; i < XB; ++i)
+            store_chunk(xs + std::min(base + tid + i * NT, nchunks - 1), xv[i]);
     }
     if (tid == 0) xs[nchunks] = uint4{0, 0, 0, 0};
     __syncthreads();
@@ -1527,19 +1544,24 @@ __global__ __launch_bounds__(NT) void gemv_lds_kernel(
             dot_chunk(S{}, src[jj], xs[c < nchunks ? c : nchunks], accs);
         }
     };
-    int b = 0;
-    for (; b + 2 < nbatch; b += 2) {
-        load(wn, b + 1);
-        comp(wa, b);
-        load(wa, b + 2);
-        comp(wn, b + 1);
-    }
-    if (b + 1 < nbatch) {
-        load(wn, b + 1);
-        comp(wa, b);
-        comp(wn, b + 1);
+    if constexpr (ONE) {
+        comp(wa, 0);
     } else {
-        comp(wa, b);
+        uint4 wn[JB];
+        int b = 0;
+        for (; b + 2 < nbatch; b += 2) {
+            load(wn, b + 1);
+            comp(wa, b);
+            load(wa, b + 2);
+            comp(wn, b + 1);
+        }
+        if (b + 1 < nbatch) {
+            load(wn, b + 1);
+            comp(wa, b);
+            comp(wn, b + 1);
+        } else {
+            comp(wa, b);
+        }
     }
     float acc = (accs[0] + accs[1]) + (accs[2] + accs[3]);
     acc = segment_sum<CW>(acc);
@@ -1580,9 +1602,9 @@ __global__ __launch_bounds__(NT) void gemv_tiled_kernel(
         const int tc = std::min(TC, nchunks - c0);            // chunks in this tile
         const int nbatch = ((tc + 63) / 64 + JB - 1) / JB;    // wave-uniform
         const uint4* xt = x + c0;
-        uint4 xv[XPER];
+        u32x4 xv[XPER];
 #pragma unroll
-        for (int i = 0; i < XPER; ++i) xv[i] = xt[std::min(tid + i * NT, tc - 1)];
+        for (int i = 0; i < XPER; ++i) xv[i] = load_chunk(xt + std::min(tid + i * NT, tc - 1));
         __builtin_amdgcn_sched_barrier(0);
         uint4 wa[JB], wn[JB];
         auto load = [&](uint4 (&dst)[JB], int b) {
@@ -1596,7 +1618,7 @@ __global__ __launch_bounds__(NT) void gemv_tiled_kernel(
         load(wa, 0);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int i = 0; i < XPER; ++i) xs[std::min(tid + i * NT, tc - 1)] = xv[i];
+        for (int i = 0; i < XPER; ++i) store_chunk(xs + std::min(tid + i * NT, tc - 1), xv[i]);
         if (tid == 0) xs[TC] = uint4{0, 0, 0, 0};
         __syncthreads();
         auto comp = [&](const uint4 (&src)[JB], int b) {
@@ -2333,18 +2355,19 @@ template <typename S>
 using GemvFn = void (*)(const uint4*, const uint4*, S*, int, int);
 
 template <typename S, int NT, int JB>
-GemvFn<S> gemv_instance_nt(int cw) {
-    if (cw == 16) return &gemv_lds_kernel<S, 16, NT, JB>;
-    if (cw == 32) return &gemv_lds_kernel<S, 32, NT, JB>;
-    if (cw == 64) return &gemv_lds_kernel<S, 64, NT, JB>;
+GemvFn<S> gemv_instance_nt(int cw, int j) {
+    if (j > JB) return cw == 64 ? &gemv_lds_kernel<S, 64, NT, JB, false> : nullptr;
+    if (cw == 16) return &gemv_lds_kernel<S, 16, NT, JB, true>;
+    if (cw == 32) return &gemv_lds_kernel<S, 32, NT, JB, true>;
+    if (cw == 64) return &gemv_lds_kernel<S, 64, NT, JB, true>;
     return nullptr;
 }
 
 template <typename S, int NT>
 GemvFn<S> gemv_instance_jb(int cw, int j) {
-    if (j <= 2) return gemv_instance_nt<S, NT, 2>(cw);
-    if (j <= 4) return gemv_instance_nt<S, NT, 4>(cw);
-    return gemv_instance_nt<S, NT, kGemvBatch>(cw);
+    if (j <= 2) return gemv_instance_nt<S, NT, 2>(cw, j);
+    if (j <= 4) return gemv_instance_nt<S, NT, 4>(cw, j);
+    return gemv_instance_nt<S, NT, kGemvBatch>(cw, j);
 }
 
 template <typename S>
