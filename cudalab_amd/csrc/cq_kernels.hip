@@ -107,13 +107,17 @@ __device__ __forceinline__ float segment_sum(float v) {
 // mapping).  Against one contiguous range of rows per XCD, where the eight
 // XCDs read eight far-apart regions at once (us per call, HBM-cold, runs of
 // 32): INT8 8192^2 13.5 -> 12.0, INT4 8192^2 8.1 -> 7.5, INT8 11008x4096 9.05
-// -> 8.4, INT4 32000x4096 13.3 -> 12.4, FP16 32000x4096 42.1 -> 41.1; launches
-// under 10 MB level.  Runs of 8 and 64 are up to 3% slower than 32 in places.
+// -> 8.4, INT4 32000x4096 13.3 -> 12.4; launches under 10 MB level.  Runs of 8 and 64 are up to 3% slower than 32 in places.
 // Where waves hold at most two chunks per lane, runs of 64: such a launch of
 // 512 workgroups is over in 3.4 us and 1-3% slower with runs of 32 (INT4
-// 4096^2, FP16 4096x1024).  The INT8 and FP16/FP32 K-tiled kernels keep one
-// run per XCD (INT8 4096x28672 20.7 us against 20.9, FP16 3000x65536 66.9
-// against 68.0): their waves live long enough to drift apart.
+// 4096^2).  The INT8 K-tiled and the FP16/FP32 kernels keep one run per XCD
+// (INT8 4096x28672 20.7 us against 20.9, FP16 3000x65536 66.9 against 68.0):
+// their waves live long enough to drift apart.  For the FP kernels it also
+// keeps the first pass over weights not read before short: FP16 32000x4096
+// 59.2 us against 66.7 with runs of 32, FP32 4096x11008 43.0 against 51.1
+// (each XCD then meets an eighth of the pages).  Later passes: FP16
+// 32000x4096 41.5 against 40.6, 4096^2 6.86 against 6.60, FP32 4096x11008
+// 31.6 against 32.1.
 constexpr uint32_t kXcdRun = 32;
 constexpr uint32_t kXcdAll = 1u << 24;   // one run per XCD
 // Run for waves that load `chunks` 16-byte chunks per lane in all.
@@ -1502,7 +1506,7 @@ __global__ __launch_bounds__(NT) void gemv_lds_kernel(
 #pragma unroll
     for (int i = 0; i < XB; ++i) xv[i] = load_chunk(x + std::min(tid + i * NT, nchunks - 1));
     __builtin_amdgcn_sched_barrier(0);
-    const uint32_t blk = xcd_block<xcd_run(JB)>();
+    const uint32_t blk = xcd_block<kXcdAll>();
     const int64_t row =
         (static_cast<int64_t>(blk) * (NT >> 6) + (tid >> 6)) * SLOTS + slot;
     const uint32_t rowc = static_cast<uint32_t>(std::min<int64_t>(row, n - 1));
