@@ -2360,7 +2360,8 @@ using GemvFn = void (*)(const uint4*, const uint4*, S*, int, int);
 
 template <typename S, int NT, int JB>
 GemvFn<S> gemv_instance_nt(int cw, int j) {
-    if (j > JB) return cw == 64 ? &gemv_lds_kernel<S, 64, NT, JB, false> : nullptr;
+    if constexpr (JB == kGemvBatch)    // only the longest batch is taken more than once
+        if (j > JB) return cw == 64 ? &gemv_lds_kernel<S, 64, NT, JB, false> : nullptr;
     if (cw == 16) return &gemv_lds_kernel<S, 16, NT, JB, true>;
     if (cw == 32) return &gemv_lds_kernel<S, 32, NT, JB, true>;
     if (cw == 64) return &gemv_lds_kernel<S, 64, NT, JB, true>;
