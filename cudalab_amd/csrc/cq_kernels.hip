@@ -1484,10 +1484,20 @@ __device__ __forceinline__ void store_chunk(uint4* p, u32x4 v) {
     *reinterpret_cast<u32x4*>(p) = v;
 }
 
-// JB: chunks per lane per register batch, the smaller of kGemvBatch and
-// the lane's chunk count rounded up to a power of two (a batch longer than
-// the row would load and multiply padding).  ONE: the row is one batch; the
-// kernel is then a third of the size, and all of x is staged in one pass.
+// Chunk w of a row, or zero where the lane re-read it past the row end.  x is
+// zero there too, but 0 * w is NaN where w is infinite.  Only LDS reads may be
+// scheduled across: moved ahead of the earlier chunks' products, the selects
+// wait for every load of the batch (FP16 1024x4096 3.34 us, 3.23 in place;
+// without selects 3.22; FP16 4096^2 5.11 against 5.07, 4096x11008 17.2 against 17.1).
+__device__ __forceinline__ uint4 if_in_row(bool in, const uint4& w) {
+    __builtin_amdgcn_sched_barrier(0x100);
+    return {in ? w.x : 0u, in ? w.y : 0u, in ? w.z : 0u, in ? w.w : 0u};
+}
+
+// JB: chunks per lane per register batch.  ONE: the row is one batch of
+// exactly the lane's chunk count (only its last chunk can pass the row end);
+// the kernel is then a third of the size, and all of x is staged in one pass.
+// Longer rows go in batches of kGemvBatch.
 template <typename S, int CW, int NT, int JB, bool ONE>
 __global__ __launch_bounds__(NT) void gemv_lds_kernel(
         const uint4* __restrict__ w,   // [n][nchunks] 16-byte chunks
@@ -1515,11 +1525,13 @@ __global__ __launch_bounds__(NT) void gemv_lds_kernel(
     const int nbatch = ((nchunks + CW - 1) / CW + JB - 1) / JB;
 
     uint4 wa[JB];
+    constexpr int kOneFull = ONE ? JB - 1 : 0;   // chunks that are inside the row
     auto load = [&](uint4 (&dst)[JB], int b) {
 #pragma unroll
         for (int jj = 0; jj < JB; ++jj) {
             const int c = col + CW * (b * JB + jj);
-            const uint32_t cl = static_cast<uint32_t>(c < nchunks ? c : nchunks - 1);
+            const uint32_t cl =
+                static_cast<uint32_t>(jj < kOneFull || c < nchunks ? c : nchunks - 1);
             dst[jj] = *reinterpret_cast<const uint4*>(wb + (rowc * wrow_bytes + cl * 16u));
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -1541,30 +1553,43 @@ __global__ __launch_bounds__(NT) void gemv_lds_kernel(
     __syncthreads();
 
     float accs[4] = {0.f, 0.f, 0.f, 0.f};
-    auto comp = [&](const uint4 (&src)[JB], int b) {
+    // The first FULL chunks of the batch are inside the row in every lane.
+    // CLAMP: their x is read as if they might not be (in the loop below the
+    // compiler then keeps two LDS reads in flight: FP16 1024x16384 5.59 us
+    // against 5.70).  The last whole chunk stays behind the others for the
+    // reason given at if_in_row.
+    auto comp = [&]<int FULL, bool CLAMP = false>(const uint4 (&src)[JB], int b) {
 #pragma unroll
         for (int jj = 0; jj < JB; ++jj) {
             const int c = col + CW * (b * JB + jj);
-            dot_chunk(S{}, src[jj], xs[c < nchunks ? c : nchunks], accs);
+            if (!CLAMP && jj == FULL - 1) __builtin_amdgcn_sched_barrier(0x100);
+            if (jj < FULL) dot_chunk(S{}, src[jj], xs[CLAMP ? std::min(c, nchunks) : c], accs);
+            else dot_chunk(S{}, if_in_row(c < nchunks, src[jj]), xs[std::min(c, nchunks)], accs);
         }
     };
     if constexpr (ONE) {
-        comp(wa, 0);
+        comp.template operator()<kOneFull>(wa, 0);
     } else {
         uint4 wn[JB];
+        // a last batch that the row fills needs no selects (FP32 1024x4096
+        // 4.54 us against 4.65; a row of one batch is no faster for it)
+        auto last = [&](const uint4 (&src)[JB], int b) {
+            if (nchunks % (CW * JB) == 0) comp.template operator()<JB>(src, b);
+            else comp.template operator()<0>(src, b);
+        };
         int b = 0;
         for (; b + 2 < nbatch; b += 2) {
             load(wn, b + 1);
-            comp(wa, b);
+            comp.template operator()<JB, true>(wa, b);
             load(wa, b + 2);
-            comp(wn, b + 1);
+            comp.template operator()<JB, true>(wn, b + 1);
         }
         if (b + 1 < nbatch) {
             load(wn, b + 1);
-            comp(wa, b);
-            comp(wn, b + 1);
+            comp.template operator()<JB, true>(wa, b);
+            last(wn, b + 1);
         } else {
-            comp(wa, b);
+            last(wa, b);
         }
     }
     float acc = (accs[0] + accs[1]) + (accs[2] + accs[3]);
@@ -1602,8 +1627,7 @@ __global__ __launch_bounds__(NT) void gemv_tiled_kernel(
     const char* wrow = reinterpret_cast<const char*>(w) +
                        rowc * (static_cast<uint32_t>(nchunks) * 16u);
     float accs[4] = {0.f, 0.f, 0.f, 0.f};
-    for (int c0 = 0; c0 < nchunks; c0 += TC) {
-        const int tc = std::min(TC, nchunks - c0);            // chunks in this tile
+    auto tile = [&]<bool PARTIAL>(int c0, int tc) {           // chunks [c0, c0 + tc)
         const int nbatch = ((tc + 63) / 64 + JB - 1) / JB;    // wave-uniform
         const uint4* xt = x + c0;
         u32x4 xv[XPER];
@@ -1629,7 +1653,8 @@ __global__ __launch_bounds__(NT) void gemv_tiled_kernel(
 #pragma unroll
             for (int jj = 0; jj < JB; ++jj) {
                 const int c = col + 64 * (b * JB + jj);
-                dot_chunk(S{}, src[jj], xs[c < tc ? c : TC], accs);
+                if (PARTIAL) dot_chunk(S{}, if_in_row(c < tc, src[jj]), xs[c < tc ? c : TC], accs);
+                else dot_chunk(S{}, src[jj], xs[c], accs);
             }
         };
         for (int b = 0; b < nbatch; b += 2) {
@@ -1641,7 +1666,10 @@ __global__ __launch_bounds__(NT) void gemv_tiled_kernel(
             }
         }
         __syncthreads();
-    }
+    };
+    int c0 = 0;
+    for (; c0 + TC <= nchunks; c0 += TC) tile.template operator()<false>(c0, TC);
+    if (c0 < nchunks) tile.template operator()<true>(c0, nchunks - c0);
     float acc = (accs[0] + accs[1]) + (accs[2] + accs[3]);
     acc = segment_sum<64>(acc);
     if (col == 63 && row < n) fp_store(y + row, acc);
@@ -2358,27 +2386,28 @@ namespace {
 template <typename S>
 using GemvFn = void (*)(const uint4*, const uint4*, S*, int, int);
 
-template <typename S, int NT, int JB>
-GemvFn<S> gemv_instance_nt(int cw, int j) {
-    if constexpr (JB == kGemvBatch)    // only the longest batch is taken more than once
-        if (j > JB) return cw == 64 ? &gemv_lds_kernel<S, 64, NT, JB, false> : nullptr;
-    if (cw == 16) return &gemv_lds_kernel<S, 16, NT, JB, true>;
-    if (cw == 32) return &gemv_lds_kernel<S, 32, NT, JB, true>;
-    if (cw == 64) return &gemv_lds_kernel<S, 64, NT, JB, true>;
-    return nullptr;
-}
-
 template <typename S, int NT>
-GemvFn<S> gemv_instance_jb(int cw, int j) {
-    if (j <= 2) return gemv_instance_nt<S, NT, 2>(cw, j);
-    if (j <= 4) return gemv_instance_nt<S, NT, 4>(cw, j);
-    return gemv_instance_nt<S, NT, kGemvBatch>(cw, j);
+GemvFn<S> gemv_instance_nt(int cw, int j) {
+    if (cw == 16 && j == 1) return &gemv_lds_kernel<S, 16, NT, 1, true>;
+    if (cw == 32 && j == 1) return &gemv_lds_kernel<S, 32, NT, 1, true>;
+    if (cw != 64 || j < 1) return nullptr;
+    switch (j) {
+    case 1: return &gemv_lds_kernel<S, 64, NT, 1, true>;
+    case 2: return &gemv_lds_kernel<S, 64, NT, 2, true>;
+    case 3: return &gemv_lds_kernel<S, 64, NT, 3, true>;
+    case 4: return &gemv_lds_kernel<S, 64, NT, 4, true>;
+    case 5: return &gemv_lds_kernel<S, 64, NT, 5, true>;
+    case 6: return &gemv_lds_kernel<S, 64, NT, 6, true>;
+    case 7: return &gemv_lds_kernel<S, 64, NT, 7, true>;
+    case kGemvBatch: return &gemv_lds_kernel<S, 64, NT, kGemvBatch, true>;
+    default: return &gemv_lds_kernel<S, 64, NT, kGemvBatch, false>;
+    }
 }
 
 template <typename S>
 GemvFn<S> gemv_instance(int cw, int j, int block) {
-    if (block == 512) return gemv_instance_jb<S, 512>(cw, j);
-    if (block == kBlock) return gemv_instance_jb<S, kBlock>(cw, j);
+    if (block == 512) return gemv_instance_nt<S, 512>(cw, j);
+    if (block == kBlock) return gemv_instance_nt<S, kBlock>(cw, j);
     return nullptr;
 }
 
@@ -2395,7 +2424,7 @@ hipError_t prepare_gemv_t(const Plan& p, const void* w, const void* x, void* y,
                     static_cast<const uint4*>(x), static_cast<S*>(y),
                     static_cast<int>(n), nchunks);
     const GemvFn<S> fn = gemv_instance<S>(p.cw, p.j, p.block);
-    if (fn == nullptr) return hipErrorInvalidConfiguration;
+    if (fn == nullptr || !lds_chunks_ok(p, nchunks)) return hipErrorInvalidConfiguration;
     return bind(L, fn, p.grid, p.block, static_cast<uint32_t>((nchunks + 1) * 16),
                 static_cast<const uint4*>(w), static_cast<const uint4*>(x),
                 static_cast<S*>(y), static_cast<int>(n), nchunks);
