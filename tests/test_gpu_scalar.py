@@ -8,7 +8,6 @@ gives the oracle's value bit for bit; operands at several offsets.
 """
 from __future__ import annotations
 
-import numpy as np
 import pytest
 import torch
 
@@ -71,22 +70,61 @@ def test_int4_scalar_exact(ext4, k):
             _same_bits(y, want, f"n={n} k={k} w+{woff} x+{xoff}")
 
 
-def test_scalar_nonfinite(ext8, cuda):
-    """Inf and NaN operands meet exactly their own products: the rounds that
-    re-read a row's last chunk add nothing."""
+# whole chunks of a row, none a multiple of 64, so that lanes of the last round
+# re-read the row's last chunk: one wave per row; two; four; four with batches
+# of two chunks, whose last batch passes the wave's last round
+PART_ROUNDS = (40, 72, 136, 324, 1028, 1156, 2116)
+
+
+def _signs(like):
+    """+1, -1, +1, ... down the rows."""
+    return torch.tensor([1, -1] * 4, device="cuda").to(like)
+
+
+@pytest.mark.parametrize("chunks", PART_ROUNDS)
+@pytest.mark.parametrize("per", [32, 16, 8, 4], ids=["int4", "int8", "f16", "f32"])
+def test_scalar_nonfinite(ext4, ext8, cuda, per, chunks):
+    """Rounds that re-read a row's last chunk add nothing of it, whichever of
+    its operands is infinite: a zero in the place of the other one would make
+    the row NaN instead of +-Inf.  A NaN stays in its own row."""
     from cudalab_amd.build import build
-    k = 64 * 16 + 5
-    wq, s, x = _q8_exact(8, k, seed=3)
-    wq[wq == 0] = 1
-    x.fill_(1.0)
-    x[k - 1] = float("inf")             # in the partial chunk
-    wq[:, k - 1] = torch.tensor([1, -1] * 4, dtype=torch.int8, device="cuda")
-    announce("qgemv scalar inf x")
-    y = ext8.forward("qgemv_baseline", wq, s, x)
-    assert torch.equal(y, torch.tensor([np.inf, -np.inf] * 4, device="cuda").half())
-    extg = build("gemv")
-    W = torch.ones(8, k, dtype=torch.float16, device="cuda")
-    W[:, 64 * 16 - 1] = float("inf")    # last element of the last whole chunk
-    announce("gemv scalar inf W")
-    y = extg.forward("gemv_baseline", W, torch.ones(k, dtype=torch.float16, device="cuda"))
-    assert torch.isposinf(y).all()
+    inf, nan, n = float("inf"), float("nan"), 8
+    assert chunks % 64
+    k = chunks * per
+    last = k - per                       # the last whole chunk starts here
+    x = torch.ones(k, dtype=torch.float32 if per == 4 else torch.float16, device="cuda")
+    xi = x.clone()
+    xi[last + 1] = inf
+    want = inf * _signs(torch.float32)
+    if per == 32:
+        # weights +1 (0x11) or -1 (0xFF) by row; the last group's scale infinite
+        W = torch.where(_signs(torch.float32) > 0, 0x11, 0xFF).to(torch.uint8)
+        W = W.unsqueeze(1).repeat(1, k // 2)
+        s = torch.full((n, k // 128), 0.25, dtype=torch.float16, device="cuda")
+        si, sn = s.clone(), s.clone()
+        si[:, -1], sn[3, -1] = inf, nan
+        calls = {"x": (W, s, xi), "scale": (W, si, x), "nan": (W, sn, x)}
+        run = lambda *a: ext4.forward("int4gemv_baseline", *a)     # noqa: E731
+    elif per == 16:
+        W = _signs(torch.int8).unsqueeze(1).repeat(1, k)
+        s = torch.full((n,), 0.25, device="cuda")
+        sn = s.clone()
+        sn[3] = nan
+        calls = {"x": (W, s, xi), "scale": (W, torch.full_like(s, inf), x), "nan": (W, sn, x)}
+        run = lambda *a: ext8.forward("qgemv_baseline", *a)        # noqa: E731
+    else:
+        W = (0.25 * _signs(x.dtype)).unsqueeze(1).repeat(1, k)
+        Wi, Wn = W.clone(), W.clone()
+        Wi[:, last + 1] = inf * _signs(x.dtype)
+        Wn[3, last + 1] = nan
+        calls = {"x": (W, xi), "W": (Wi, x), "nan": (Wn, x)}
+        run = lambda *a: build("gemv").forward("gemv_baseline", *a)  # noqa: E731
+    for what, args in calls.items():
+        announce(f"scalar non-finite {what} per={per} k={k}")
+        y = run(*args).float()
+        if what == "nan":
+            finite = (0.25 * k * _signs(torch.float32)).to(x.dtype).float()
+            assert torch.isnan(y[3]) and torch.equal(y[:3], finite[:3]) \
+                and torch.equal(y[4:], finite[4:]), (what, y)
+        else:
+            assert torch.equal(y, want), (what, y)
