@@ -526,7 +526,7 @@ def test_timeline_by_workgroup_ranks_workgroups_sharing_a_cu():
     run on XCD x; blocks 4x, 4x+2 share one CU and 4x+1, 4x+3 another): the
     one that starts later on its CU passes its barrier later; by_workgroup
     must see it, keying a CU by its XCD and hardware id (the XCD map must
-    invert the kernels' XCD-contiguous block mapping)."""
+    invert the kernels' block mapping)."""
     import numpy as np
     from cudalab_amd.evaluator.timeline import by_workgroup, xcd_of_logical_block
     assert list(xcd_of_logical_block(16)) == [x for x in range(8) for _ in range(2)]
@@ -562,3 +562,39 @@ def test_timeline_by_workgroup_constant_starts_give_nan_correlation():
     assert g["barrier_first_on_cu_us"] == pytest.approx(1.0)
     assert g["barrier_second_on_cu_us"] is None
     assert math.isnan(g["corr_start_barrier"])
+
+
+@pytest.mark.parametrize("run", [32, 64])
+@pytest.mark.parametrize("grid", [1, 7, 10, 255, 256, 257, 300, 512, 519, 600, 1025, 1376])
+def test_timeline_xcd_map_inverts_the_kernels_block_map(grid, run):
+    """Workgroup b runs on XCD b % 8 and computes the logical block that the
+    kernels' mapping gives it, restated here forwards: the XCDs take runs of
+    `run` blocks side by side, the rest past the last whole set of runs in one
+    range each.  Grids within one set of runs, of whole sets and past them."""
+    from cudalab_amd.evaluator.timeline import by_workgroup, xcd_of_logical_block
+    import numpy as np
+    want = np.full(grid, -1)
+    for b in range(grid):
+        base = b // (8 * run) * (8 * run)
+        span, xcd = min(grid - base, 8 * run), b % 8
+        logical = base + xcd * (span // 8) + min(xcd, span % 8) + (b - base) // 8
+        assert want[logical] == -1
+        want[logical] = xcd
+    assert np.array_equal(xcd_of_logical_block(grid, run), want)
+    if grid < 512:
+        return
+    # by_workgroup takes the run: XCD x's workgroups pass their barrier at 1 + x us
+    a = np.zeros((3, grid, 8), dtype=np.int64)
+    a[:, :, 0] = 1000
+    a[:, :, 1] = 1100 + 100 * want
+    a[:, :, 5] = np.arange(grid)
+    g = by_workgroup(a, 100.0, 1, skip=0.0, run=run)
+    assert g["barrier_by_xcd_us"] == pytest.approx([1.0 + x for x in range(8)])
+
+
+@pytest.mark.parametrize("j,r,run", [(1, 1, 64), (2, 1, 64), (1, 2, 64), (3, 1, 32),
+                                     (2, 2, 32), (8, 1, 32)])
+def test_timeline_xcd_run_of_a_plan(j, r, run):
+    """Runs of 64 where a wave loads at most two chunks per lane, else 32."""
+    from cudalab_amd.evaluator.timeline import xcd_run
+    assert xcd_run({"j": str(j), "r": str(r)}) == run
