@@ -107,17 +107,18 @@ __device__ __forceinline__ float segment_sum(float v) {
 // mapping).  Against one contiguous range of rows per XCD, where the eight
 // XCDs read eight far-apart regions at once (us per call, HBM-cold, runs of
 // 32): INT8 8192^2 13.5 -> 12.0, INT4 8192^2 8.1 -> 7.5, INT8 11008x4096 9.05
-// -> 8.4, INT4 32000x4096 13.3 -> 12.4; launches under 10 MB level.  Runs of 8 and 64 are up to 3% slower than 32 in places.
-// Where waves hold at most two chunks per lane, runs of 64: such a launch of
-// 512 workgroups is over in 3.4 us and 1-3% slower with runs of 32 (INT4
-// 4096^2).  The INT8 K-tiled and the FP16/FP32 kernels keep one run per XCD
-// (INT8 4096x28672 20.7 us against 20.9, FP16 3000x65536 66.9 against 68.0):
-// their waves live long enough to drift apart.  For the FP kernels it also
-// keeps the first pass over weights not read before short: FP16 32000x4096
-// 59.2 us against 66.7 with runs of 32, FP32 4096x11008 43.0 against 51.1
-// (each XCD then meets an eighth of the pages).  Later passes: FP16
-// 32000x4096 41.5 against 40.6, 4096^2 6.86 against 6.60, FP32 4096x11008
-// 31.6 against 32.1.
+// -> 8.4, INT4 32000x4096 13.3 -> 12.4; launches under 10 MB level.  Runs of
+// 8 and 64 are up to 3% slower than 32 in places.  Where waves hold at most
+// two chunks per lane, runs of 64: such a launch of 512 workgroups is over in
+// 3.4 us and 1-3% slower with runs of 32 (INT4 4096^2).  The INT8 K-tiled
+// kernel keeps one run per XCD (4096x28672 20.7 us against 20.9).
+// So do the FP16/FP32 kernels, for the first pass over weights not read
+// before: FP16 32000x4096 57.5 us against 66.2 with runs of 32, FP32
+// 4096x11008 43.0 against 50.6 (why was not established).  Later passes pay
+// for it at most sizes, one run against runs of 32 (us per call from a graph):
+// FP16 4096^2 7.20, 6.90; 11008x4096 16.4, 16.1; 32000x4096 43.9, 42.9;
+// 4096x11008 17.2, 17.4; FP32 4096^2 13.1, 12.9; 5120x1600 6.90, 6.63;
+// 4096x11008 33.3, 33.7; rows of 14000 elements and more level.
 constexpr uint32_t kXcdRun = 32;
 constexpr uint32_t kXcdAll = 1u << 24;   // one run per XCD
 // Run for waves that load `chunks` 16-byte chunks per lane in all.
@@ -146,16 +147,26 @@ __device__ __forceinline__ uint32_t xcd_block() { return xcd_block<RUN>(blockIdx
 // sets: batch b + 1 is in flight while batch b is summed (its loads are
 // unconditional, see gemv_lds_kernel).  The k % E elements past the last whole
 // chunk go one per lane.  Four accumulators per lane keep the FMA chains as
-// short as one element per thread of a 256-thread workgroup would; the shares of a row meet in LDS and are added in wave order.  Chunks
-// past the row end are re-read in bounds and not summed (no zero operand
-// stands in for them, so an infinite scale or x meets no extra product).
+// short as one element per thread of a 256-thread workgroup would; the shares
+// of a row meet in LDS and are added in wave order.  Chunks past the row end
+// are re-read in bounds and not summed (no zero operand stands in for them, so
+// an infinite scale or x meets no extra product).
 //
-// Bound by memory.  With one element per load and one workgroup per row (the
-// form before) the memory system was idle: INT8 4001x4099 (16 MB) 12.2 us,
-// now 6.1; FP16 4096^2 off alignment 18.3 us, now 7.5.  What is left of the
-// distance to the aligned kernels (INT8 4096^2 4.4 us) is the loads that
-// start off a 4-byte boundary: the same INT8 4096^2 call on this kernel is
-// 5.3 us with W 4 or 8 bytes off, 6.0 with W 1 or 2 bytes off.
+// With one element per load and one workgroup per row (the form before) the
+// memory system was idle: INT8 4096^2 with W and x off alignment 18.2 us, now
+// 7.45; FP16 18.3, now 10.8.  What bounds it now, by us per call (HBM-cold)
+// on aligned data; W 1 to 3 bytes off (FP16: 2); x 2 bytes off; both; and the
+// LDS kernels on the aligned data:
+//   INT4 4096^2      4.7   4.9   6.4   7.15    3.4
+//   INT4 11008x4096  9.1   9.2  13.1  15.2     5.8
+//   INT8 4096^2      5.1   5.9   5.9   7.45    4.3
+//   INT8 11008x4096 10.7  12.3  12.1  16.3     8.5
+//   FP16 4096^2      7.1   9.2   7.5  10.8     6.9
+//   FP16 11008x4096 15.0  20.8  16.3  25.1    15.6
+// On aligned data FP16 is bound by memory (6.0 TB/s at 11008x4096), INT4 by
+// its per-element arithmetic (2.6 TB/s), INT8 (4.2 TB/s) lies between.  Off
+// alignment the unaligned loads themselves cost the difference; W or x off by
+// 4 or 8 bytes costs nothing.
 
 __device__ __forceinline__ uint4 load16_any(const char* p) {
     uint4 v;
@@ -1465,17 +1476,18 @@ __device__ __forceinline__ void dot_chunk(float, const uint4& w,
 // runs with a bounded register budget.  The loop's loads are unconditional (the
 // last batch is peeled): after a load under a condition the compiler no longer
 // knows how many are in flight and waits for all of them before it multiplies.
-// FP16 4096x11008 17.5 -> 16.8 us, 1000x30000 16.6 -> 15.7, 32000x4096 41.1 ->
-// 40.3, FP32 2000x14000 23.7 -> 22.9.  (The K-tiled kernel below keeps its
-// conditional loads: four batches a tile between two barriers gain nothing,
-// 3000x65536 67.2 us against 66.6.)
+// FP16 4096x11008 17.4 -> 17.2 us (a graph's calls), 1000x30000 13.8 -> 13.6,
+// FP32 2000x14000 26.9 -> 26.7, others level.  (The K-tiled kernel below keeps
+// its conditional loads: four batches a tile between two barriers gained
+// nothing.)
 constexpr int kGemvBatch = 8;
 
 // A chunk of x on its way to LDS is held as a vector: a uint4 that is only
 // copied is forwarded from x to LDS as one memory copy, which moves the load
-// behind the weight loads, and the barrier then waits for all of them (FP16
-// 4096^2 7.2 us that way, 6.5 with x first; 1024x4096 3.43, 2.88; 1000x30000
-// 15.7, 13.0; FP32 1000x30000 on the K-tiled kernel 33.5, 23.9).
+// behind the weight loads, and the barrier then waits for all of them (us per
+// call of a graph that way and with x first: FP16 1024x4096 3.57, 3.23;
+// 1024x16384 8.17, 7.89; FP32 1024x4096 5.16, 4.55; 4096^2 level; on the K-tiled
+// kernel FP16 3000x65536 121, 70.7, FP32 1000x30000 37.6, 24.0).
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ u32x4 load_chunk(const uint4* p) {
     return *reinterpret_cast<const u32x4*>(p);
@@ -1487,8 +1499,9 @@ __device__ __forceinline__ void store_chunk(uint4* p, u32x4 v) {
 // Chunk w of a row, or zero where the lane re-read it past the row end.  x is
 // zero there too, but 0 * w is NaN where w is infinite.  Only LDS reads may be
 // scheduled across: moved ahead of the earlier chunks' products, the selects
-// wait for every load of the batch (FP16 1024x4096 3.34 us, 3.23 in place;
-// without selects 3.22; FP16 4096^2 5.11 against 5.07, 4096x11008 17.2 against 17.1).
+// wait for every load of the batch (us per call of a graph: FP16 1024x4096
+// 3.34, in place 3.23, without the selects 3.22; in place and without them
+// 4096^2 7.22, 7.16, 4096x11008 17.2, 17.1).
 __device__ __forceinline__ uint4 if_in_row(bool in, const uint4& w) {
     __builtin_amdgcn_sched_barrier(0x100);
     return {in ? w.x : 0u, in ? w.y : 0u, in ? w.z : 0u, in ? w.w : 0u};
@@ -1555,8 +1568,8 @@ __global__ __launch_bounds__(NT) void gemv_lds_kernel(
     float accs[4] = {0.f, 0.f, 0.f, 0.f};
     // The first FULL chunks of the batch are inside the row in every lane.
     // CLAMP: their x is read as if they might not be (in the loop below the
-    // compiler then keeps two LDS reads in flight: FP16 1024x16384 5.59 us
-    // against 5.70).  The last whole chunk stays behind the others for the
+    // compiler then keeps two LDS reads in flight: FP16 1024x16384 7.90 us
+    // against 8.05).  The last whole chunk stays behind the others for the
     // reason given at if_in_row.
     auto comp = [&]<int FULL, bool CLAMP = false>(const uint4 (&src)[JB], int b) {
 #pragma unroll
@@ -2416,7 +2429,8 @@ hipError_t prepare_gemv_t(const Plan& p, const void* w, const void* x, void* y,
                           int64_t n, int64_t k, Launch* L) {
     if (p.kind == kScalar)
         return bind(L, scalar_instance<GemvScalar<S>>(p), p.grid, p.block, 0,
-                    static_cast<const char*>(w), nullptr, static_cast<const char*>(x), static_cast<S*>(y), static_cast<int>(n), k);
+                    static_cast<const char*>(w), nullptr, static_cast<const char*>(x),
+                    static_cast<S*>(y), static_cast<int>(n), k);
     const int nchunks = static_cast<int>(k * static_cast<int64_t>(sizeof(S)) / 16);
     if (p.kind == kTiled)
         return bind(L, p.block == 512 ? gemv_tiled_kernel<S, 512> : gemv_tiled_kernel<S, kBlock>,

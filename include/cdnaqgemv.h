@@ -37,9 +37,15 @@
  *
  * Vector contract (checked on the host before every launch): the vectorized
  * kernels need w and x 16-byte aligned and k % 32 == 0 (int4gemv),
- * k % 16 == 0 (qgemv), k % 8 == 0 (gemv fp16) or k % 4 == 0 (gemv fp32).  Inputs that miss it are never rejected: they run on
- * the scalar kernel of the `*_baseline` variant, so their output is
- * bit-identical to that variant's.
+ * k % 16 == 0 (qgemv), k % 8 == 0 (gemv fp16) or k % 4 == 0 (gemv fp32).
+ * Inputs that miss it are never rejected: they run on the scalar kernel of
+ * the `*_baseline` variant, so their output is bit-identical to that
+ * variant's.
+ *
+ * Non-finite inputs: NaN or Inf in w (gemv) or x meets only its own products,
+ * on every variant.  The scales of int4gemv and qgemv are taken to be finite,
+ * as in the reference (int4gemv_common.h:60-67): the int4gemv vector kernels
+ * may give NaN where *_baseline gives Inf for an infinite group scale.
  *
  * Errors: every entry point returns a CQ_* status; on error nothing was
  * launched (or, for CQ_ERR_HIP, the HIP runtime refused the launch) and

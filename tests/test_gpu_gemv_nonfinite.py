@@ -1,9 +1,9 @@
-"""GPU test of infinite operands in the FP16/FP32 LDS and K-tiled kernels.
-Lanes past the row end re-read the row's last chunk of W and sum nothing of
-it: an Inf there meets only its own x, and the row is +-Inf as on the scalar
-kernel, not NaN (0 * Inf).  Chunk counts that leave lanes, chunks of a lane
-or both past the row end, in one batch, in the last of several, and in the
-last tile; full rows beside them."""
+"""GPU tests of infinite operands in the vector kernels.  Lanes past the row
+end re-read the row's last chunk of W and sum nothing of it: an Inf there
+(FP16/FP32 W) or in x meets only its own product, and the row is +-Inf as on
+the scalar kernel, not NaN (0 * Inf).  Chunk counts that leave lanes, chunks of
+a lane or both past the row end, in one batch, in the last of several, and in
+the last tile; full rows beside them."""
 from __future__ import annotations
 
 import pytest
@@ -40,3 +40,23 @@ def test_infinite_operands(cuda, dtype, per, chunks):
     for v in ("gemv_cdna4", "gemv_lds_tiled", "gemv_baseline"):
         announce(f"gemv inf x {v} {dtype} k={k}")
         assert torch.equal(ext.forward(v, Ws, x), want), v
+
+
+@pytest.mark.parametrize("k", [128, 256, 640, 2048, 2176, 4096, 11008, 16384, 16512, 28672, 35072])
+@pytest.mark.parametrize("op", ["int4gemv", "qgemv"])
+def test_infinite_x_of_quantized_weights(cuda, op, k):
+    ext, n = build(op), 12
+    sign = torch.tensor([1, -1] * (n // 2), device="cuda")
+    if op == "int4gemv":
+        W = torch.where(sign > 0, 0x11, 0xFF).to(torch.uint8).unsqueeze(1).repeat(1, k // 2)
+        s = torch.full((n, k // 128), 0.25, dtype=torch.float16, device="cuda")
+    else:
+        W = sign.to(torch.int8).unsqueeze(1).repeat(1, k)
+        s = torch.full((n,), 0.25, device="cuda")
+    want = (float("inf") * sign).half()
+    for at in (0, k - 1):
+        x = torch.ones(k, dtype=torch.float16, device="cuda")
+        x[at] = float("inf")
+        for v in ext.variants():
+            announce(f"{op} inf x {v} k={k} at {at}")
+            assert torch.equal(ext.forward(v, W, s, x), want), (v, at)
