@@ -855,10 +855,14 @@ def quantize_finite(op: str, W: torch.Tensor, rcp: bool = True
     """quantize_int4 / quantize_q8 and whether all of W is finite, known once
     the call returns: the kernel sets a word of pinned host memory, and the
     call waits for the current stream and reads it.  The word is this call's
-    own, so calls from several threads do not meet."""
+    own, so calls from several threads do not meet, and is given up only
+    behind the wait, also where the call is interrupted."""
+    stream = torch.cuda.current_stream(W.device)
     flag = torch.zeros(1, dtype=torch.int32, device="cpu", pin_memory=True)
-    q, scale = _quantize(op, W, rcp, flag)
-    torch.cuda.current_stream(W.device).synchronize()
+    try:
+        q, scale = _quantize(op, W, rcp, flag)
+    finally:
+        stream.synchronize()
     return q, scale, flag.item() == 0
 
 

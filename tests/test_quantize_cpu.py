@@ -331,3 +331,40 @@ def test_quantize_path_selection(op, w, out, n, k, fast):
 def test_quantize_path_selection_rejects_other_ops():
     lib = _capi.load()
     assert lib.cq_quantize_vectorized(_capi.CQ_OP_GEMV_F16, 0x1000, 0x1000, 1, 8) == -1
+
+
+def test_nonfinite_word_outlives_an_interrupted_call(monkeypatch):
+    """The kernel may still write the pinned word when the call is interrupted
+    behind the launch (a signal handler that raises): the call waits for the
+    stream before it lets the word go, else the next owner of that memory
+    finds it overwritten."""
+    import weakref
+
+    import torch
+
+    from cudalab_amd import ext
+
+    class Word:
+        pass
+
+    words, waited = [], []
+
+    class Stream:
+        def synchronize(self):
+            waited.append(words[0]() is not None)
+
+    def zeros(*args, **kw):
+        word = Word()
+        words.append(weakref.ref(word))
+        return word
+
+    def interrupted(op, W, rcp, flag):
+        raise KeyboardInterrupt
+
+    monkeypatch.setattr(torch, "zeros", zeros)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: Stream())
+    monkeypatch.setattr(ext, "_quantize", interrupted)
+    W = torch.empty(1, 128, dtype=torch.float16)
+    with pytest.raises(KeyboardInterrupt):
+        ext.quantize_finite("int4gemv", W)
+    assert waited == [True]
