@@ -857,12 +857,11 @@ def quantize_finite(op: str, W: torch.Tensor, rcp: bool = True
     call waits for the current stream and reads it.  The word is this call's
     own, so calls from several threads do not meet, and is given up only
     behind the wait, also where the call is interrupted."""
-    stream = torch.cuda.current_stream(W.device)
     flag = torch.zeros(1, dtype=torch.int32, device="cpu", pin_memory=True)
     try:
         q, scale = _quantize(op, W, rcp, flag)
     finally:
-        stream.synchronize()
+        torch.cuda.current_stream(W.device).synchronize()
     return q, scale, flag.item() == 0
 
 
