@@ -1623,7 +1623,11 @@ __global__ __launch_bounds__(NT) void gemv_lds_kernel(
 constexpr int kGemvTileJ = 4 * kGemvBatch;    // 32 chunks per lane per tile
 constexpr uint32_t kGemvTileLds = (kGemvTileJ * 64 + 1) * 16u;   // 32,784 B
 
-template <typename S, int NT>
+// ONE: the row is shorter than a tile (gemv_lds_tiled at such k, or weights of
+// 4 GiB and more).  A kernel of its own, as the loop over whole tiles takes 168
+// VGPRs with fp16 and halves the workgroups per CU: FP16 4096^2 7.6 us against
+// 8.8.
+template <typename S, int NT, bool ONE>
 __global__ __launch_bounds__(NT) void gemv_tiled_kernel(
         const uint4* __restrict__ w,   // [n][nchunks] 16-byte chunks
         const uint4* __restrict__ x,   // [nchunks] 16-byte chunks
@@ -1680,9 +1684,13 @@ __global__ __launch_bounds__(NT) void gemv_tiled_kernel(
         }
         __syncthreads();
     };
-    int c0 = 0;
-    for (; c0 + TC <= nchunks; c0 += TC) tile.template operator()<false>(c0, TC);
-    if (c0 < nchunks) tile.template operator()<true>(c0, nchunks - c0);
+    if constexpr (ONE) {
+        tile.template operator()<true>(0, nchunks);
+    } else {
+        int c0 = 0;
+        for (; c0 + TC <= nchunks; c0 += TC) tile.template operator()<false>(c0, TC);
+        if (c0 < nchunks) tile.template operator()<true>(c0, nchunks - c0);
+    }
     float acc = (accs[0] + accs[1]) + (accs[2] + accs[3]);
     acc = segment_sum<64>(acc);
     if (col == 63 && row < n) fp_store(y + row, acc);
@@ -2418,6 +2426,12 @@ GemvFn<S> gemv_instance_nt(int cw, int j) {
 }
 
 template <typename S>
+GemvFn<S> gemv_tiled_instance(int block, bool one) {
+    if (block == 512) return one ? &gemv_tiled_kernel<S, 512, true> : &gemv_tiled_kernel<S, 512, false>;
+    return one ? &gemv_tiled_kernel<S, kBlock, true> : &gemv_tiled_kernel<S, kBlock, false>;
+}
+
+template <typename S>
 GemvFn<S> gemv_instance(int cw, int j, int block) {
     if (block == 512) return gemv_instance_nt<S, 512>(cw, j);
     if (block == kBlock) return gemv_instance_nt<S, kBlock>(cw, j);
@@ -2433,8 +2447,7 @@ hipError_t prepare_gemv_t(const Plan& p, const void* w, const void* x, void* y,
                     static_cast<S*>(y), static_cast<int>(n), k);
     const int nchunks = static_cast<int>(k * static_cast<int64_t>(sizeof(S)) / 16);
     if (p.kind == kTiled)
-        return bind(L, p.block == 512 ? gemv_tiled_kernel<S, 512> : gemv_tiled_kernel<S, kBlock>,
-                    p.grid, p.block, kGemvTileLds, static_cast<const uint4*>(w),
+        return bind(L, gemv_tiled_instance<S>(p.block, nchunks < kGemvTileJ * 64), p.grid, p.block, kGemvTileLds, static_cast<const uint4*>(w),
                     static_cast<const uint4*>(x), static_cast<S*>(y),
                     static_cast<int>(n), nchunks);
     const GemvFn<S> fn = gemv_instance<S>(p.cw, p.j, p.block);
